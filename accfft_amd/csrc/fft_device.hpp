@@ -145,7 +145,7 @@ __device__ __forceinline__ void dft16(cpx<T>* v) {
   }
 }
 
-// Odd prime R in {3, 5, 7} by the symmetric pair form:
+// Odd prime R in {3, 5, 7, 11, 13} by the symmetric pair form:
 //   X[q]   = v0 + sum_r a_r cos(2 pi r q/R) + SIGN*i sum_r b_r sin(2 pi r q/R)
 //   X[R-q] = v0 + sum_r a_r cos(.)          - SIGN*i sum_r b_r sin(.)
 // with a_r = v[r] + v[R-r], b_r = v[r] - v[R-r].
@@ -177,6 +177,44 @@ template <> struct OddConst<7> {
     const double t[7] = {0.0, 0.78183148246802980871, 0.97492791218182360702,
                          0.43388373911755812048, -0.43388373911755812048,
                          -0.97492791218182360702, -0.78183148246802980871};
+    return t[m];
+  }
+};
+
+template <> struct OddConst<11> {
+  static __device__ __forceinline__ double c(int m) {
+    const double t[11] = {
+        1.00000000000000000000, 0.84125353283118116886, 0.41541501300188642549,
+        -0.14231483827328514046, -0.65486073394528506413, -0.95949297361449738990,
+        -0.95949297361449738990, -0.65486073394528506407, -0.14231483827328514024,
+        0.41541501300188642568, 0.84125353283118116892};
+    return t[m];
+  }
+  static __device__ __forceinline__ double s(int m) {
+    const double t[11] = {
+        0.0, 0.54064081745559758210, 0.90963199535451837142, 0.98982144188093273236,
+        0.75574957435425828370, 0.28173255684142969765, -0.28173255684142969773,
+        -0.75574957435425828376, -0.98982144188093273241, -0.90963199535451837136,
+        -0.54064081745559758199};
+    return t[m];
+  }
+};
+template <> struct OddConst<13> {
+  static __device__ __forceinline__ double c(int m) {
+    const double t[13] = {
+        1.00000000000000000000, 0.88545602565320989587, 0.56806474673115580249,
+        0.12053668025532305325, -0.35460488704253562600, -0.74851074817110109868,
+        -0.97094181742605202719, -0.97094181742605202719, -0.74851074817110109863,
+        -0.35460488704253562600, 0.12053668025532305346, 0.56806474673115580238,
+        0.88545602565320989609};
+    return t[m];
+  }
+  static __device__ __forceinline__ double s(int m) {
+    const double t[13] = {
+        0.0, 0.46472317204376854566, 0.82298386589365639458, 0.99270887409805399284,
+        0.93501624268541482345, 0.66312265824079520232, 0.23931566428755776695,
+        -0.23931566428755776706, -0.66312265824079520243, -0.93501624268541482345,
+        -0.99270887409805399278, -0.82298386589365639469, -0.46472317204376854531};
     return t[m];
   }
 };
@@ -411,6 +449,7 @@ struct DynSched {
   int n;
   int nst;
   int rad[20];
+  int roots;  // LDS elements after the tile's buffers for a prime stage's roots (0: none)
 };
 
 // Flat butterfly index b -> (line, j).  Layout Z: line stride LS, element
@@ -439,6 +478,11 @@ struct LayZ {
   __device__ __forceinline__ void map(int b, int nb, float rnb, int& line, int& j) const {
     line = fdivmod(b, nb, rnb, j);
   }
+  // (butterfly u, output q) of a prime stage: threads walk q fastest, so a
+  // wavefront reads the same inputs and writes neighbouring outputs
+  __device__ __forceinline__ void map_q(int b, int Q, float rq, int& u, int& q) const {
+    u = fdivmod(b, Q, rq, q);
+  }
 };
 struct LayS {
   int w;
@@ -446,6 +490,12 @@ struct LayS {
   __device__ __forceinline__ void map(int b, int nb, float rnb, int& line, int& j) const {
     j = b >> (__ffs(w) - 1);  // w is a power of two
     line = b & (w - 1);
+  }
+  // columns fastest, then q
+  __device__ __forceinline__ void map_q(int b, int Q, float rq, int& u, int& q) const {
+    const int sh = __ffs(w) - 1;
+    const int j = fdivmod(b >> sh, Q, rq, q);
+    u = (j << sh) | (b & (w - 1));
   }
 };
 
@@ -478,41 +528,95 @@ __device__ __forceinline__ void dstage(const cpx<T>* src, cpx<T>* dst, int N, in
   }
 }
 
-// Generic radix (any R, O(R^2) per butterfly) straight from LDS.
+// Prime radix R > 13, O(R^2) per butterfly, by the symmetric pair form of
+// dft_odd: a first sweep applies the stage's twiddles and replaces
+// x[r], x[R-r] by a_r = x[r] + x[R-r], b_r = x[r] - x[R-r] in place (src is
+// scratch from here on), a second one forms each output pair q, R-q from
+// the H = (R-1)/2 products a_r cos, b_r sin.  `roots`: R LDS elements for
+// exp(-2 pi i m / R), nullptr when the tile leaves no room (the roots are
+// then read from the length-N table).  A thread takes two values of q, so
+// that each a_r, b_r it reads serves two outputs; the root index r q mod R
+// is kept by an addition and a conditional subtraction.  (One thread per
+// output with all R terms, a table read and two 64-bit remainders per term
+// took 1.3 ms for the 61-point x pass of a 61 x 45 x 70 FP64 transform,
+// whose arithmetic is below a microsecond.)
 template <typename T, int SIGN, class Lay>
-__device__ __forceinline__ void dstage_generic(const cpx<T>* src, cpx<T>* dst, int N, int R,
-                                               int NS, int nlines, const Lay& lay,
-                                               const cpx<T>* __restrict__ twg) {
-  const int NB = N / R;
-  const int total = nlines * NB;
+__device__ void dstage_prime(cpx<T>* src, cpx<T>* dst, int N, int R, int NS, int nlines,
+                             const Lay& lay, const cpx<T>* __restrict__ twg, cpx<T>* roots) {
+  const int NB = N / R, H = (R - 1) / 2;
   const int tstep = N / (NS * R);
-  const int rstep = N / R;
   const float rnb = 1.0f / (float)NB, rns = 1.0f / (float)NS;
-  for (int b = threadIdx.x; b < total; b += blockDim.x) {
-    int line, j, k;
-    lay.map(b, NB, rnb, line, j);
-    (void)fdivmod(j, NS, rns, k);
-    const int base = (j - k) * R + k;
-    for (int q = 0; q < R; ++q) {
-      cpx<T> acc = {(T)0, (T)0};
-      for (int r = 0; r < R; ++r) {
-        const long m = ((long)r * k * tstep + (long)((r * q) % R) * rstep) % N;
-        const cpx<T> w = twg[m];
-        const cpx<T> x = src[lay.addr(line, j + r * NB)];
-        const cpx<T> t = (SIGN < 0) ? cmul(x, w) : cmulc(x, w);
-        acc = cadd(acc, t);
+  if (roots != nullptr)
+    for (int m = threadIdx.x; m < R; m += blockDim.x) roots[m] = twg[m * NB];
+  {
+    const int nj = nlines * NB, total = nj * H;
+    const float rnj = 1.0f / (float)nj;
+    for (int b = threadIdx.x; b < total; b += blockDim.x) {
+      int u, line, j, k;
+      const int r = fdivmod(b, nj, rnj, u) + 1;
+      lay.map(u, NB, rnb, line, j);
+      (void)fdivmod(j, NS, rns, k);
+      const int p1 = lay.addr(line, j + r * NB), p2 = lay.addr(line, j + (R - r) * NB);
+      cpx<T> x = src[p1], y = src[p2];
+      if (NS > 1) {
+        const cpx<T> wx = twg[r * k * tstep], wy = twg[(R - r) * k * tstep];
+        x = (SIGN < 0) ? cmul(x, wx) : cmulc(x, wx);
+        y = (SIGN < 0) ? cmul(y, wy) : cmulc(y, wy);
       }
-      dst[lay.addr(line, base + q * NS)] = acc;
+      src[p1] = cadd(x, y);
+      src[p2] = csub(x, y);
+    }
+  }
+  __syncthreads();
+  const int Q = (H + 2) / 2;  // values of q: u and u + Q
+  const int nj = nlines * NB, total = nj * Q;
+  const float rq = 1.0f / (float)Q;
+  for (int b = threadIdx.x; b < total; b += blockDim.x) {
+    int q1, u, line, j, k;
+    lay.map_q(b, Q, rq, u, q1);
+    lay.map(u, NB, rnb, line, j);
+    (void)fdivmod(j, NS, rns, k);
+    const int q2 = q1 + Q <= H ? q1 + Q : 0;
+    const cpx<T> v0 = src[lay.addr(line, j)];
+    cpx<T> c1 = v0, c2 = v0, s1 = {(T)0, (T)0}, s2 = {(T)0, (T)0};
+    int m1 = 0, m2 = 0;
+    for (int r = 1; r <= H; ++r) {
+      const cpx<T> x = src[lay.addr(line, j + r * NB)], y = src[lay.addr(line, j + (R - r) * NB)];
+      m1 += q1;
+      m1 = m1 >= R ? m1 - R : m1;
+      m2 += q2;
+      m2 = m2 >= R ? m2 - R : m2;
+      const cpx<T> w1 = roots != nullptr ? roots[m1] : twg[m1 * NB];
+      const cpx<T> w2 = roots != nullptr ? roots[m2] : twg[m2 * NB];
+      c1.x += x.x * w1.x;
+      c1.y += x.y * w1.x;
+      s1.x += y.x * w1.y;  // -sin
+      s1.y += y.y * w1.y;
+      c2.x += x.x * w2.x;
+      c2.y += x.y * w2.x;
+      s2.x += y.x * w2.y;
+      s2.y += y.y * w2.y;
+    }
+    const int base = (j - k) * R + k;
+    // w.y = -sin, so the SIGN * i sin term is mul_si<-SIGN>
+    const cpx<T> t1 = mul_si<-SIGN>(s1), t2 = mul_si<-SIGN>(s2);
+    dst[lay.addr(line, base + q1 * NS)] = cadd(c1, t1);
+    if (q1 > 0) dst[lay.addr(line, base + (R - q1) * NS)] = csub(c1, t1);
+    if (q2 > 0) {
+      dst[lay.addr(line, base + q2 * NS)] = cadd(c2, t2);
+      dst[lay.addr(line, base + (R - q2) * NS)] = csub(c2, t2);
     }
   }
 }
 
 // Runs the whole transform; data starts in a, the returned pointer holds the
 // result (a or b).  Caller must __syncthreads() before; returns after a
-// barrier.
-template <typename T, int SIGN, class Lay>
+// barrier.  PRIMES: the schedule may hold radices 11, 13 and larger primes
+// (kernels of their own: with these stages in the kernel every other length
+// ran 2-6 % slower, 384^3 FP32 round trip 899 -> 915 us).
+template <typename T, int SIGN, bool PRIMES, class Lay>
 __device__ cpx<T>* dyn_fft(cpx<T>* a, cpx<T>* b, const DynSched& sc, int nlines,
-                           const Lay& lay, const cpx<T>* __restrict__ twg) {
+                           const Lay& lay, const cpx<T>* __restrict__ twg, cpx<T>* roots) {
   int NS = 1;
   const int N = sc.n;
   for (int s = 0; s < sc.nst; ++s) {
@@ -526,7 +630,13 @@ __device__ cpx<T>* dyn_fft(cpx<T>* a, cpx<T>* b, const DynSched& sc, int nlines,
       case 8: dstage<T, 8, SIGN>(a, b, N, NS, nlines, lay, twg); break;
       case 9: dstage<T, 9, SIGN>(a, b, N, NS, nlines, lay, twg); break;
       case 16: dstage<T, 16, SIGN>(a, b, N, NS, nlines, lay, twg); break;
-      default: dstage_generic<T, SIGN>(a, b, N, R, NS, nlines, lay, twg); break;
+      default:
+        if constexpr (PRIMES) {
+          if (R == 11) dstage<T, 11, SIGN>(a, b, N, NS, nlines, lay, twg);
+          else if (R == 13) dstage<T, 13, SIGN>(a, b, N, NS, nlines, lay, twg);
+          else dstage_prime<T, SIGN>(a, b, N, R, NS, nlines, lay, twg, roots);
+        }
+        break;
     }
     __syncthreads();
     cpx<T>* t = a;

@@ -183,7 +183,8 @@ __device__ __forceinline__ void stage_twiddles(cpx<T>* dst, const cpx<T>* __rest
 }
 
 // -------------------------------------------------------------- engines
-// N > 0: static engine; N == 0: dynamic engine.
+// N > 0: static engine; N == 0: dynamic engine, N == -1: dynamic engine for
+// lengths with a prime factor above 7.
 template <typename T, int N, int NT, int SIGN, int SPLIT = 0, int LINES = 256 / NT, int PAD = 0,
           typename PRE = NoPre>
 __device__ __forceinline__ cpx<T>* zrun(cpx<T>* A, cpx<T>* B, const FftArgs<T>& a,
@@ -195,7 +196,9 @@ __device__ __forceinline__ cpx<T>* zrun(cpx<T>* A, cpx<T>* B, const FftArgs<T>& 
     return A;
   } else {
     LayZ lay{a.sc.n};
-    return dyn_fft<T, SIGN>(A, B, a.sc, lpw, lay, a.tw);
+    cpx<T>* lo = A < B ? A : B;
+    return dyn_fft<T, SIGN, (N < 0)>(A, B, a.sc, lpw, lay, a.tw,
+                            a.sc.roots ? lo + 2 * lpw * a.sc.n : nullptr);
   }
 }
 
@@ -209,7 +212,9 @@ __device__ __forceinline__ cpx<T>* srun(cpx<T>* A, cpx<T>* B, const FftArgs<T>& 
     return A;
   } else {
     LayS lay{w_dyn};
-    return dyn_fft<T, SIGN>(A, B, a.sc, w_dyn, lay, a.tw);
+    cpx<T>* lo = A < B ? A : B;
+    return dyn_fft<T, SIGN, (N < 0)>(A, B, a.sc, w_dyn, lay, a.tw,
+                            a.sc.roots ? lo + 2 * w_dyn * a.sc.n : nullptr);
   }
 }
 

@@ -69,23 +69,47 @@ inline bool static_length(int n) {
 
 inline bool pair_mode(int mode) { return mode == M_R2C || mode == M_C2R || mode == M_DERIV; }
 
-inline int dyn_lines(int n) {
+// Tiles of the dynamic engine.  A launch of few blocks is bound by the
+// latency of one block's stages, so tiles are halved while the launch has
+// fewer than dyn_blocks blocks (one for each CU) and a tile keeps whole
+// 64-byte row segments (strided) or one line (z).
+constexpr int64_t dyn_blocks = 256;
+inline int dyn_lines(int n, int64_t units) {
   int l = 2048 / n;
   if (l < 1) l = 1;
   if (l > 64) l = 64;
+  while (l > 1 && (units + l - 1) / l < dyn_blocks) l = (l + 1) / 2;
   return l;
 }
 // Strided dynamic tiles: the widest power-of-two column count whose buffer
 // stays within 32 KiB (4096 FP32 / 2048 FP64 elements; two buffers per
 // workgroup).  FP64 tiles of 4096 elements (128 KiB per workgroup, one per
 // CU) ran 768^3 in 22.4 ms against 18.9 ms.
-inline int dyn_cols(int n, size_t csz) {
+inline int dyn_cols(int n, size_t csz, int64_t units) {
   int w = 1;
   while (w * 2 <= 64 && (size_t)w * 2 * n * csz <= 32768) w *= 2;
+  while ((size_t)w * csz > 64 && (units + w - 1) / w < dyn_blocks) w /= 2;
   return w;
 }
 inline size_t dyn_z_lds(int n, int lpw, size_t csz) { return 2 * (size_t)lpw * n * csz; }
 inline size_t dyn_s_lds(int n, int w, size_t csz) { return 2 * (size_t)w * n * csz; }
+
+// Bytes of LDS for the roots of the schedule's largest prime stage (R > 13),
+// 0 when it has none or they do not fit beside the tile.
+inline size_t dyn_roots(DynSched& sc, size_t shm, size_t csz) {
+  int r = 0;
+  for (int s = 0; s < sc.nst; ++s)
+    if (sc.rad[s] > 16 && sc.rad[s] > r) r = sc.rad[s];
+  sc.roots = shm + r * csz <= 160 * 1024 ? r : 0;
+  return sc.roots * csz;
+}
+
+// Whether the schedule has a prime factor above 7.
+inline bool dyn_primes(const DynSched& sc) {
+  for (int s = 0; s < sc.nst; ++s)
+    if (sc.rad[s] > 9 && sc.rad[s] != 16) return true;
+  return false;
+}
 
 template <typename T, int N, int ZT = 256>
 hipError_t launch_z_n(int mode, int sign, FftArgs<T>& a, int64_t grid, size_t shm,
@@ -129,17 +153,23 @@ inline void dyn_lds_attrs() {
   if (done) return;
   done = true;
   const int cap = 160 * 1024;
-  (void)hipFuncSetAttribute((const void*)zfft_kernel<T, 0, M_C2C, -1>, hipFuncAttributeMaxDynamicSharedMemorySize, cap);
-  (void)hipFuncSetAttribute((const void*)zfft_kernel<T, 0, M_C2C, +1>, hipFuncAttributeMaxDynamicSharedMemorySize, cap);
-  (void)hipFuncSetAttribute((const void*)zfft_kernel<T, 0, M_R2C, -1>, hipFuncAttributeMaxDynamicSharedMemorySize, cap);
-  (void)hipFuncSetAttribute((const void*)zfft_kernel<T, 0, M_C2R, +1>, hipFuncAttributeMaxDynamicSharedMemorySize, cap);
-  (void)hipFuncSetAttribute((const void*)zfft_kernel<T, 0, M_DERIV, -1>, hipFuncAttributeMaxDynamicSharedMemorySize, cap);
-  (void)hipFuncSetAttribute((const void*)sfft_kernel<T, 0, M_C2C, -1>, hipFuncAttributeMaxDynamicSharedMemorySize, cap);
-  (void)hipFuncSetAttribute((const void*)sfft_kernel<T, 0, M_C2C, +1>, hipFuncAttributeMaxDynamicSharedMemorySize, cap);
-  (void)hipFuncSetAttribute((const void*)sfft_kernel<T, 0, M_R2C, -1>, hipFuncAttributeMaxDynamicSharedMemorySize, cap);
-  (void)hipFuncSetAttribute((const void*)sfft_kernel<T, 0, M_C2R, +1>, hipFuncAttributeMaxDynamicSharedMemorySize, cap);
-  (void)hipFuncSetAttribute((const void*)sfft_kernel<T, 0, M_DERIV, -1>, hipFuncAttributeMaxDynamicSharedMemorySize, cap);
-  (void)hipFuncSetAttribute((const void*)sfft_kernel<T, 0, M_MULT, -1>, hipFuncAttributeMaxDynamicSharedMemorySize, cap);
+#define AFFT_CAP(K) (void)hipFuncSetAttribute((const void*)K, hipFuncAttributeMaxDynamicSharedMemorySize, cap)
+#define AFFT_CAPS(N)                      \
+  AFFT_CAP((zfft_kernel<T, N, M_C2C, -1>)); \
+  AFFT_CAP((zfft_kernel<T, N, M_C2C, +1>)); \
+  AFFT_CAP((zfft_kernel<T, N, M_R2C, -1>)); \
+  AFFT_CAP((zfft_kernel<T, N, M_C2R, +1>)); \
+  AFFT_CAP((zfft_kernel<T, N, M_DERIV, -1>)); \
+  AFFT_CAP((sfft_kernel<T, N, M_C2C, -1>)); \
+  AFFT_CAP((sfft_kernel<T, N, M_C2C, +1>)); \
+  AFFT_CAP((sfft_kernel<T, N, M_R2C, -1>)); \
+  AFFT_CAP((sfft_kernel<T, N, M_C2R, +1>)); \
+  AFFT_CAP((sfft_kernel<T, N, M_DERIV, -1>)); \
+  AFFT_CAP((sfft_kernel<T, N, M_MULT, -1>))
+  AFFT_CAPS(0);
+  AFFT_CAPS(-1);
+#undef AFFT_CAPS
+#undef AFFT_CAP
 }
 
 // Strided C2C tiles of half the LDS (32 KiB: twice the workgroups per CU,
@@ -460,17 +490,23 @@ hipError_t launch_fft(bool strided, int mode, int sign, FftArgs<T> a, const Axis
   a.tw = tab.tw_full;
   dyn_lds_attrs<T>();
   if (strided) {
-    const int w = dyn_cols(n, csz);
-    const size_t shm = dyn_s_lds(n, w, csz);
+    const int w = dyn_cols(n, csz, units);
+    size_t shm = dyn_s_lds(n, w, csz);
     if (shm > 160 * 1024) return hipErrorNotSupported;
+    shm += dyn_roots(a.sc, shm, csz);
     a.lpw = w;
-    return launch_s_n<T, 0>(mode, sign, a, (units + w - 1) / w, shm, st);
+    const int64_t grid = (units + w - 1) / w;
+    return dyn_primes(a.sc) ? launch_s_n<T, -1>(mode, sign, a, grid, shm, st)
+                            : launch_s_n<T, 0>(mode, sign, a, grid, shm, st);
   } else {
-    const int l = dyn_lines(n);
-    const size_t shm = dyn_z_lds(n, l, csz);
+    const int l = dyn_lines(n, units);
+    size_t shm = dyn_z_lds(n, l, csz);
     if (shm > 160 * 1024) return hipErrorNotSupported;
+    shm += dyn_roots(a.sc, shm, csz);
     a.lpw = l;
-    return launch_z_n<T, 0>(mode, sign, a, (units + l - 1) / l, shm, st);
+    const int64_t grid = (units + l - 1) / l;
+    return dyn_primes(a.sc) ? launch_z_n<T, -1>(mode, sign, a, grid, shm, st)
+                            : launch_z_n<T, 0>(mode, sign, a, grid, shm, st);
   }
 }
 

@@ -165,11 +165,29 @@ inline int static_sched(int n, int R[3], int split = 0) {
 #undef AFFT_SCHED
 }
 
-inline DynSched dyn_sched(int n) {
+// tile: the schedule of an LDS tile (primes above 13 first, where their
+// stage needs no twiddles; radices 11 and 13 in registers); otherwise the
+// global radix passes of fft_long.hpp.
+inline DynSched dyn_sched(int n, bool tile = false) {
   DynSched s{};
   s.n = n;
   s.nst = 0;
   int m = n;
+  if (tile) {
+    int c = n;
+    for (int f : {2, 3, 5, 7, 11, 13})
+      while (c % f == 0) c /= f;
+    for (int f = 17; c > 1 && s.nst < 20;) {
+      if ((long)f * f > c) f = c;
+      if (c % f) {
+        f += 2;
+        continue;
+      }
+      s.rad[s.nst++] = f;
+      c /= f;
+      m /= f;
+    }
+  }
   // 9 before 3: a power of three takes half the LDS passes
   const int pref[] = {16, 8, 4, 2, 9, 3, 5, 7};
   for (int f : pref)
