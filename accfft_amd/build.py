@@ -36,17 +36,26 @@ FLAGS = [
 if os.environ.get("ACCFFT_AMD_SWEEP", "0") not in ("", "0"):
     # measurement build: tile / order overrides read from the environment
     FLAGS.append("-DACCFFT_AMD_SWEEP")
-SOURCES = ["fft_f32.hip", "fft_f64.hip", "fft_split.hip", "transpose.hip", "capi.hip"]
+# (source, object name, defines); the mixed-radix kernels are one source
+# compiled per part of fft_mix_list.hpp and precision
+MIX_PARTS = 6
+UNITS = [(s, os.path.splitext(s)[0], [])
+         for s in ("fft_f32.hip", "fft_f64.hip", "fft_split.hip")]
+UNITS += [("fft_mix.hip", f"fft_mix_{t}_{p}",
+           [f"-DAFFT_T={t}", f"-DAFFT_PART={p}", f"-DAFFT_PART_LIST=AFFT_MIX_{p}"])
+          for p in range(MIX_PARTS) for t in ("float", "double")]
+UNITS += [(s, os.path.splitext(s)[0], []) for s in ("transpose.hip", "capi.hip")]
 
 
-def _compile(src: str) -> str:
-    obj = os.path.join(OBJ, os.path.splitext(src)[0] + ".o")
-    cmd = [HIPCC, *FLAGS, "-c", os.path.join(CSRC, src), "-o", obj]
+def _compile(unit) -> str:
+    src, name, defs = unit
+    obj = os.path.join(OBJ, name + ".o")
+    cmd = [HIPCC, *FLAGS, *defs, "-c", os.path.join(CSRC, src), "-o", obj]
     r = subprocess.run(cmd, capture_output=True, text=True)
     noise = "is not a recognized feature for this target"
     err = "\n".join(l for l in r.stderr.splitlines() if noise not in l)
     if r.returncode != 0:
-        raise RuntimeError(f"hipcc failed on {src}:\n{err}")
+        raise RuntimeError(f"hipcc failed on {name}:\n{err}")
     if err.strip():
         sys.stderr.write(err + "\n")
     return obj
@@ -72,9 +81,9 @@ def build_dropin_example() -> str:
 
 def build(verbose: bool = True) -> str:
     os.makedirs(OBJ, exist_ok=True)
-    jobs = min(len(SOURCES), int(os.environ.get("MAX_JOBS", "4")) or 1)
+    jobs = min(len(UNITS), int(os.environ.get("MAX_JOBS", "8")) or 1)
     with cf.ThreadPoolExecutor(max_workers=jobs) as ex:
-        objs = list(ex.map(_compile, SOURCES))
+        objs = list(ex.map(_compile, UNITS))
     tmp = LIB + ".tmp"
     cmd = [HIPCC, f"--offload-arch={ARCH}", "-shared", "-fPIC", *objs, "-o", tmp]
     r = subprocess.run(cmd, capture_output=True, text=True)

@@ -6,6 +6,7 @@
 
 #include "fft_kernels.hpp"
 #include "fft_long.hpp"
+#include "fft_mix_list.hpp"
 
 namespace afft {
 
@@ -34,6 +35,7 @@ struct AxisTab {
   const cpx<T>* tw_split = nullptr;   // per-stage table of the split schedule
   const cpx<T>* tw_sub = nullptr;     // per-stage table of length n/16 (two-level tiles)
   const cpx<T>* tw_subw = nullptr;    // the same for the SCHED_WIDE schedule
+  const cpx<T>* tw_mix = nullptr;     // per-stage table of the mixed-radix kernels (mix_part >= 0)
   // strided C2C configuration picked by the plan's MEASURE tuning: -1 the
   // built-in rule, -2 one-level tiles, v >= 0 two-level variant S4Cfg<T, n, v>
   int s4v = -1;
@@ -353,6 +355,21 @@ hipError_t launch_s4(int sign, FftArgs<T>& a, const AxisTab<T>& tab, hipStream_t
   }
 }
 
+// Adjacent real columns of a strided M_DERIV pass as complex columns: even
+// column counts and strides, aligned pointers.
+template <typename T>
+inline bool pair_columns(FftArgs<T>& a) {
+  if ((a.nlines | a.C | a.Din | a.Dout | a.Sin | a.Sout) & 1) return false;
+  if (((uintptr_t)a.in | (uintptr_t)a.out) % sizeof(cpx<T>)) return false;
+  a.nlines /= 2;
+  a.C /= 2;
+  a.Din /= 2;
+  a.Dout /= 2;
+  a.Sin /= 2;
+  a.Sout /= 2;
+  return true;
+}
+
 // Fused two-level tiles for a strided M_MULT / M_DERIV pass (FP32 512,
 // 1024, 2048); hipErrorNotSupported sends the caller to the one-level tile.
 // M_DERIV runs on the complex view of adjacent real columns, which needs
@@ -360,14 +377,7 @@ hipError_t launch_s4(int sign, FftArgs<T>& a, const AxisTab<T>& tab, hipStream_t
 template <typename T>
 hipError_t launch_s4f(int mode, FftArgs<T> a, const AxisTab<T>& tab, hipStream_t st) {
   if (mode == M_DERIV) {
-    if ((a.nlines | a.C | a.Din | a.Dout | a.Sin | a.Sout) & 1) return hipErrorNotSupported;
-    if (((uintptr_t)a.in | (uintptr_t)a.out) % sizeof(cpx<T>)) return hipErrorNotSupported;
-    a.nlines /= 2;
-    a.C /= 2;
-    a.Din /= 2;
-    a.Dout /= 2;
-    a.Sin /= 2;
-    a.Sout /= 2;
+    if (!pair_columns(a)) return hipErrorNotSupported;
   }
   a.tw = tab.tw_full;
 #define AFFT_S4F(NN)                                                                        \
@@ -392,6 +402,26 @@ hipError_t launch_s4f(int mode, FftArgs<T> a, const AxisTab<T>& tab, hipStream_t
   AFFT_S4F(2048)
 #undef AFFT_S4F
   return hipErrorNotSupported;
+}
+
+// The mixed-radix kernels (lengths of fft_mix_list.hpp): every mode but the
+// exchange-block rows, the Poisson symbols, strided real transforms and
+// derivatives of odd column counts, which stay with the run-time engine.
+template <typename T>
+hipError_t launch_mix(bool strided, int mode, int sign, FftArgs<T> a, const AxisTab<T>& tab,
+                      hipStream_t st) {
+  if (a.ishift || a.oshift) return hipErrorNotSupported;
+  if (strided && mode == M_DERIV && !pair_columns(a)) return hipErrorNotSupported;
+  if (mode == M_MULT && a.sym > SYM_INV_BIHARMONIC) return hipErrorNotSupported;
+  a.tw = tab.tw_mix;
+  const int64_t units = !strided && pair_mode(mode) ? (a.nlines + 1) / 2 : a.nlines;
+  switch (mix_part(tab.n)) {
+#define AFFT_MIX_CASE(P) \
+  case P: return mix_launch<T, P>(strided, mode, sign, a, tab.n, units, st);
+    AFFT_MIX_EACH(AFFT_MIX_CASE)
+#undef AFFT_MIX_CASE
+    default: return hipErrorNotSupported;
+  }
 }
 
 // Launch one axis pass.  strided = false: contiguous lines (z layout).
@@ -486,6 +516,10 @@ hipError_t launch_fft(bool strided, int mode, int sign, FftArgs<T> a, const Axis
       default: return hipErrorInvalidValue;
     }
 #undef AFFT_CASE
+  }
+  if (tab.tw_mix) {
+    const hipError_t e = launch_mix<T>(strided, mode, sign, a, tab, st);
+    if (e != hipErrorNotSupported) return e;
   }
   a.tw = tab.tw_full;
   dyn_lds_attrs<T>();

@@ -15,6 +15,7 @@
 
 #include "../../include/accfft_amd.h"
 #include "fft_launch.hpp"
+#include "fft_mix.hpp"
 
 struct accfft_amd_plan {
   int n[3] = {0, 0, 0};
@@ -227,7 +228,25 @@ inline std::vector<cpx<T>> static_table(int n, int split = 0) {
 template <typename T>
 inline std::vector<cpx<T>> full_table(int n) {
   std::vector<cpx<T>> tw(n > 0 ? n : 1);
-  for (int m = 0; m < n; ++m) tw[m] = host_root<T>(m, n);
+  for (int m = 0; 2 * m <= n && m < n; ++m) {
+    tw[m] = host_root<T>(m, n);
+    if (m) tw[n - m] = {tw[m].x, -tw[m].y};
+  }
+  return tw;
+}
+
+// The per-stage table of the compile-time mixed-radix schedule (fft_mix.hpp)
+// out of the length's full table.
+template <typename T>
+inline std::vector<cpx<T>> mix_table(int n, const std::vector<cpx<T>>& full) {
+  const MixSched m = mix_sched(n);
+  std::vector<cpx<T>> tw;
+  tw.reserve(mix_twn(m));
+  for (int s = 1; s < m.s; ++s) {
+    const int ns = mix_ns(m, s), step = n / (ns * m.r[s]);
+    for (int r = 1; r < m.r[s]; ++r)
+      for (int k = 0; k < ns; ++k) tw.push_back(full[r * k * step]);  // r k step < n
+  }
   return tw;
 }
 
