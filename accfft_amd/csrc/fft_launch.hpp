@@ -424,6 +424,23 @@ hipError_t launch_mix(bool strided, int mode, int sign, FftArgs<T> a, const Axis
   }
 }
 
+// Powers of two on the mixed-radix kernels.  Strided up to 256 points: one
+// or two LDS round trips instead of three or four (64^3 FP64 passes 9.0-10
+// -> 6.5-7.2 us, 256^3 FP32 x pass 29 -> 26 us, multiply 47 -> 30 us,
+// derivatives 38 -> 28 us, FP64 51 -> 47, 81 -> 54, 65-69 -> 52-56 us); 512
+// points FP64 (multiply 569 -> 423 us, derivatives 751 / 512 -> 570 / 407
+// us, C2C 401-418 -> 388-394 us) and FP32 C2C (204 / 197 -> 197 / 184 us; the
+// fused FP32 passes stay with the two-level tiles, derivatives 219 against
+// 240-250 us).  z up to 128 points (64^3 FP64 8.5 -> 6.6 us) and the FP32
+// derivative at 256 and 512 (37 -> 32, 276 -> 217 us); the other z passes are
+// faster as they are (256^3 FP64 r2c 60 against 69 us, 512^3 369 against 410
+// us).  A plan's tuned choice (s4v) comes first.
+template <typename T>
+inline bool mix_pow2(int n, bool strided, int mode) {
+  if (strided) return n <= 256 || (n == 512 && (sizeof(T) == 8 || mode == M_C2C));
+  return n <= 128 || (sizeof(T) == 4 && mode == M_DERIV && n <= 512);
+}
+
 // Launch one axis pass.  strided = false: contiguous lines (z layout).
 // Returns hipErrorNotSupported when the length does not fit one LDS tile.
 template <typename T>
@@ -435,6 +452,10 @@ hipError_t launch_fft(bool strided, int mode, int sign, FftArgs<T> a, const Axis
   const int64_t units = pair_mode(mode) ? (a.nlines + 1) / 2 : a.nlines;
   if (units <= 0) return hipSuccess;
   const size_t csz = sizeof(cpx<T>);
+  if (tab.tw_mix && tab.is_static && tab.s4v == -1 && mix_pow2<T>(n, strided, mode)) {
+    const hipError_t e = launch_mix<T>(strided, mode, sign, a, tab, st);
+    if (e != hipErrorNotSupported) return e;
+  }
   if (tab.is_static) {
     a.tw = tab.tw_static;
     int per;

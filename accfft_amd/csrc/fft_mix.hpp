@@ -1,5 +1,6 @@
 // fft_mix.hpp -- compile-time mixed-radix tiles: lengths with the prime
-// factors 2, 3, 5 and 7 that are not covered by the power-of-two kernels.
+// factors 2, 3, 5 and 7, powers of two included where they are faster than
+// the tiles of fft_kernels.hpp (mix_pow2 in fft_launch.hpp).
 //
 // A tile is L lines of N points.  N is split at compile time into two to
 // four radices of at most 16 (mix_sched); every stage is a Stockham stage
@@ -75,14 +76,15 @@ struct MixSched {
 constexpr bool mix_radix(int r) { return (r >= 2 && r <= 10) || r == 12 || (r >= 14 && r <= 16); }
 // The fewest stages whose radices are at most 16, and among those the
 // smallest largest radix (fewest registers).
-constexpr MixSched mix_sched(int n) {
+// `most`: the largest radix allowed.
+constexpr MixSched mix_search(int n, int most) {
   MixSched best{0, {1, 1, 1, 1}};
-  for (int a = 2; a <= 16 && !best.s; ++a) {
+  for (int a = 2; a <= most && !best.s; ++a) {
     if (!mix_radix(a) || n % a) continue;
     const int b = n / a;
     if (b <= a && mix_radix(b)) best = MixSched{2, {a, b, 1, 1}};
   }
-  for (int a = 2; a <= 16 && !best.s; ++a) {
+  for (int a = 2; a <= most && !best.s; ++a) {
     if (!mix_radix(a) || n % a) continue;
     for (int b = a; b >= 2 && !best.s; --b) {
       if (!mix_radix(b) || (n / a) % b) continue;
@@ -90,7 +92,7 @@ constexpr MixSched mix_sched(int n) {
       if (c <= b && c >= 2 && mix_radix(c)) best = MixSched{3, {a, b, c, 1}};
     }
   }
-  for (int a = 2; a <= 16 && !best.s; ++a) {
+  for (int a = 2; a <= most && !best.s; ++a) {
     if (!mix_radix(a) || n % a) continue;
     for (int b = a; b >= 2 && !best.s; --b) {
       if (!mix_radix(b) || (n / a) % b) continue;
@@ -102,6 +104,18 @@ constexpr MixSched mix_sched(int n) {
     }
   }
   return best;
+}
+// FP64 from 256 points: radices up to 10, more stages with half the
+// registers (256^3 derivative passes 83 -> 57 us, z r2c 93 -> 69 us, 960^3
+// strided passes 4.2 -> 3.3 ms, 768^3 1.58-1.69 -> 1.43-1.56 ms); shorter
+// lines lose by the extra exchange (240^3 derivatives 49 -> 75 us).
+template <typename T>
+constexpr MixSched mix_sched(int n) {
+  if (sizeof(T) == 8 && n >= 256) {
+    const MixSched m = mix_search(n, 10);
+    if (m.s) return m;
+  }
+  return mix_search(n, 16);
 }
 constexpr int mix_ns(const MixSched& m, int s) {  // span before stage s
   int ns = 1;
@@ -117,8 +131,7 @@ constexpr int mix_twn(const MixSched& m) { return mix_twoff(m, m.s); }
 
 // Threads per block for L lines: a multiple of the wavefront up to 512 that holds at most `most` elements a thread and leaves the fewest
 // threads without a butterfly, summed over the stages by their work.
-constexpr int mix_tpb(int n, int l, int most) {
-  const MixSched m = mix_sched(n);
+constexpr int mix_tpb(const MixSched& m, int n, int l, int most) {
   int best = 0;
   long cost = 0;
   for (int t = 64; t <= 512; t += 64) {
@@ -138,16 +151,16 @@ constexpr int mix_tpb(int n, int l, int most) {
 
 // Strided tiles: the widest power-of-two column count whose buffer stays
 // within 52 KiB (three workgroups per CU) and whose row segments are at most
-// 128 bytes, 256 for FP64 lengths of three stages.  Three-stage lengths
+// 128 bytes, 256 for FP64 lengths from 256.  Those of three stages and more
 // exchange real and imaginary parts in turn (HALF): with whole-tile
 // exchanges only two workgroups fit, 384^3 FP32 y / x passes 100 / 85 ->
 // 88 / 78 us, FP64 202 / 213 -> 175 / 188 us, and 151 / 175 us with 256-byte
 // segments (FP32: 90 / 80 us with those); 768^3 FP64 1934 / 2055 -> 1604 /
-// 1659 us, whose 64-byte segments become 128-byte ones.  Two-stage lengths
-// fit as they are (200^3 equal, FP64 with 256-byte segments 10 % slower).
+// 1659 us, whose 64-byte segments become 128-byte ones.  Lengths below 256
+// fit as they are (200^3 FP32 round trip 92 us, 97 us with HALF).
 template <typename T, int N>
 struct MixS {
-  static constexpr bool HALF = mix_sched(N).s > 2;
+  static constexpr bool HALF = mix_sched<T>(N).s > 2 && N >= 256;
   static constexpr int SEG = sizeof(T) == 8 && HALF ? 256 : 128;
   static constexpr int cols() {
     int w = 1;
@@ -156,7 +169,7 @@ struct MixS {
     return w;
   }
   static constexpr int L = cols();
-  static constexpr int TPB = mix_tpb(N, L, sizeof(T) == 4 ? 24 : 12);
+  static constexpr int TPB = mix_tpb(mix_sched<T>(N), N, L, sizeof(T) == 4 ? 24 : 12);
 };
 // Contiguous tiles: about 1152 elements and at least two lines above 256
 // points (the staged twiddle table is about one line long: 768^3 FP64 z r2c
@@ -168,7 +181,8 @@ struct MixZ {
   static constexpr int most = N > 256 ? 1152 : 2304;
   static constexpr int L0 = most / N > 2 ? most / N : 2;
   static constexpr int L = L0 > 32 ? 32 : L0;
-  static constexpr int TPB = mix_tpb(N, L, sizeof(T) == 4 ? 12 : 8);
+  static constexpr int R0 = mix_sched<T>(N).r[0], E = sizeof(T) == 4 ? 12 : 8;
+  static constexpr int TPB = mix_tpb(mix_sched<T>(N), N, L, R0 > E ? R0 : E);
 };
 
 // ---------------------------------------------------------------- engine
@@ -177,7 +191,7 @@ struct MixZ {
 // columns per CU).
 template <typename T, int N, int L, int TPB, bool STR, bool HALF = false>
 struct Mix {
-  static constexpr MixSched SC = mix_sched(N);
+  static constexpr MixSched SC = mix_sched<T>(N);
   static constexpr int S = SC.s;
   static_assert(S >= 2, "no schedule for this length");
   static constexpr int R0 = SC.r[0];

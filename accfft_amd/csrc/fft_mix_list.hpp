@@ -1,29 +1,29 @@
 // fft_mix_list.hpp -- the lengths with compile-time mixed-radix kernels
 // (fft_mix.hpp) and the interface of their launchers: every length from 18
-// to 1024 with the prime factors 2, 3 and 5, and to 512 with 7, that is not
-// a power of two.  (Longer ones and other factors run the run-time engine;
+// to 1024 with the prime factors 2, 3 and 5, and to 512 with 7, of the
+// powers of two 16 to 512.  (Longer ones and other factors run the run-time engine;
 // each length costs fourteen kernels.)  The lists are parts of about equal
 // work, compiled as translation units of their own (fft_mix.hip).
 #pragma once
 #include "fft_kernels.hpp"
 
 #define AFFT_MIX_0(X) \
-  X(18) X(28) X(45) X(60) X(81) X(105) X(135) X(162) X(196) X(240) X(280) X(324) X(378) \
+  X(16) X(18) X(28) X(45) X(60) X(81) X(105) X(135) X(162) X(196) X(240) X(280) X(324) X(378) \
   X(432) X(490) X(625) X(750) X(960)
 #define AFFT_MIX_1(X) \
-  X(20) X(30) X(48) X(63) X(84) X(108) X(140) X(168) X(200) X(243) X(288) X(336) X(384) \
+  X(32) X(20) X(30) X(48) X(63) X(84) X(108) X(140) X(168) X(200) X(243) X(288) X(336) X(384) \
   X(441) X(500) X(640) X(768) X(972)
 #define AFFT_MIX_2(X) \
-  X(21) X(35) X(49) X(70) X(90) X(112) X(144) X(175) X(210) X(245) X(294) X(343) X(392) \
+  X(64) X(21) X(35) X(49) X(70) X(90) X(112) X(144) X(175) X(210) X(245) X(294) X(343) X(392) \
   X(448) X(504) X(648) X(800) X(1000)
 #define AFFT_MIX_3(X) \
-  X(24) X(36) X(50) X(72) X(96) X(120) X(147) X(180) X(216) X(250) X(300) X(350) X(400) \
+  X(128) X(24) X(36) X(50) X(72) X(96) X(120) X(147) X(180) X(216) X(250) X(300) X(350) X(400) \
   X(450) X(540) X(675) X(810)
 #define AFFT_MIX_4(X) \
-  X(25) X(40) X(54) X(75) X(98) X(125) X(150) X(189) X(224) X(252) X(315) X(360) X(405) \
+  X(256) X(25) X(40) X(54) X(75) X(98) X(125) X(150) X(189) X(224) X(252) X(315) X(360) X(405) \
   X(480) X(576) X(720) X(864)
 #define AFFT_MIX_5(X) \
-  X(27) X(42) X(56) X(80) X(100) X(126) X(160) X(192) X(225) X(270) X(320) X(375) X(420) \
+  X(512) X(27) X(42) X(56) X(80) X(100) X(126) X(160) X(192) X(225) X(270) X(320) X(375) X(420) \
   X(486) X(600) X(729) X(900)
 #define AFFT_MIX_EACH(X) X(0) X(1) X(2) X(3) X(4) X(5)
 

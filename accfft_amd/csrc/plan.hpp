@@ -239,7 +239,7 @@ inline std::vector<cpx<T>> full_table(int n) {
 // out of the length's full table.
 template <typename T>
 inline std::vector<cpx<T>> mix_table(int n, const std::vector<cpx<T>>& full) {
-  const MixSched m = mix_sched(n);
+  const MixSched m = mix_sched<T>(n);
   std::vector<cpx<T>> tw;
   tw.reserve(mix_twn(m));
   for (int s = 1; s < m.s; ++s) {

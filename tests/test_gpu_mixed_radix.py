@@ -27,7 +27,7 @@ def test_list_is_the_rule():
             while n % p == 0:
                 n //= p
         return n
-    want = [n for n in range(18, 1025) if n & (n - 1) and
+    want = [n for n in range(16, 1025) if (n & (n - 1) or n <= 512) and
             (rest(n, (2, 3, 5)) == 1 or (n <= 512 and rest(n, (2, 3, 5, 7)) == 1))]
     assert LENGTHS == want
 
@@ -70,7 +70,7 @@ def test_transforms(dev, n, prec):
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("prec", ["f64", "f32"])
-@pytest.mark.parametrize("n", [18, 45, 70, 160, 162, 200, 384, 405, 625, 768])
+@pytest.mark.parametrize("n", [16, 18, 45, 64, 70, 160, 162, 200, 256, 384, 405, 512, 625, 768])
 def test_operators(dev, orc, n, prec):
     import torch
     import accfft_amd as af
