@@ -44,6 +44,7 @@ UNITS = [(s, os.path.splitext(s)[0], [])
 UNITS += [("fft_mix.hip", f"fft_mix_{t}_{p}",
            [f"-DAFFT_T={t}", f"-DAFFT_PART={p}", f"-DAFFT_PART_LIST=AFFT_MIX_{p}"])
           for p in range(MIX_PARTS) for t in ("float", "double")]
+UNITS += [("fft_two.hip", f"fft_two_{t}", [f"-DAFFT_T={t}"]) for t in ("float", "double")]
 UNITS += [(s, os.path.splitext(s)[0], []) for s in ("transpose.hip", "capi.hip")]
 
 

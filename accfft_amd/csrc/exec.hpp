@@ -420,11 +420,80 @@ struct Ops {
     return run_pass<T>(p, axis == 0 ? "x" : axis == 1 ? "y" : "z", strided, M_DERIV, -1, a, tab(p, axis));
   }
 
+  // ---------------------------------------------------------- two passes
+  // 1 x 1 r2c plans on power-of-two grids (fft_two.hpp).  A tuning choice on
+  // the x or y axis, or the separate z and y passes (choice -3), takes the
+  // plan back to one pass per axis.
+  static bool two(const accfft_amd_plan* p) {
+    return p->two && tab(p, 0).s4v == -1 && tab(p, 1).s4v == -1 && (ysub(p).n == 0 || p->yfuse);
+  }
+  // pass 1, real <-> half spectrum rows k1 + R n2; adjw as in the z passes
+  static int two_zy(accfft_amd_plan* p, int sign, const void* in, void* out, int adjw = 0) {
+    const int64_t N0 = p->n[0], N1 = p->n[1], N2 = p->n[2], Nh = N2 / 2 + 1, M = N1 / p->two;
+    FftArgs<T> a{};
+    a.in = in;
+    a.out = out;
+    a.idist = sign < 0 ? N2 : Nh;
+    a.odist = sign < 0 ? Nh : N2;
+    a.Din = N1 * a.idist;
+    a.Dout = N1 * a.odist;
+    a.C = M;
+    a.nlines = N0 * M;
+    a.tw = tab(p, 2).tw_full;
+    a.adjw = adjw;
+    a.xgroup = xcd_group_z();
+    auto launch = [&]() {
+      return launch_two_zy<T>(sign, p->n[2], p->two, a, tab(p, 1).tw_full, p->stream);
+    };
+    if (!p->prof) return status_of(launch());
+    char name[64];
+    snprintf(name, sizeof(name), "zyfft_%s_n%d_zy%d_%s", sign < 0 ? "r2c" : "c2r", p->n[2], p->two,
+             sizeof(T) == 4 ? "f32" : "f64");
+    return prof_launch(p, name, (double)(N0 * N1) * (N2 * sizeof(T) + Nh * sizeof(C)), launch);
+  }
+  // pass 2 over the half spectrum
+  static int two_xy(accfft_amd_plan* p, int mode, int sign, const void* in, void* out, int sym = 0,
+                    double scale = 0) {
+    const int64_t N0 = p->n[0], N1 = p->n[1], Nh = p->n[2] / 2 + 1, R = p->two;
+    if (N1 == R) {
+      if (mode == M_MULT) return x_mult(p, in, out, Nh, sym, scale);
+      return x_c2c(p, in, out, Nh, sign);
+    }
+    FftArgs<T> a{};
+    a.in = in;
+    a.out = out;
+    a.nlines = R * Nh;
+    a.Sin = a.Sout = N1 * Nh;
+    a.Din = a.Dout = R * Nh;
+    a.C = R;
+    a.Ch = Nh;
+    a.sym = sym;
+    a.scale = scale;
+    a.N0 = p->n[0];
+    a.N1 = p->n[1];
+    a.N2 = p->n[2];
+    a.tw = tab(p, 0).tw_full;
+    a.xgroup = 64;
+    a.reverse = mode == M_C2C && sign > 0;
+    auto launch = [&]() {
+      return launch_two_xy<T>(mode, sign, p->n[0], (int)(N1 / R), a, p->stream);
+    };
+    if (!p->prof) return status_of(launch());
+    char name[64];
+    snprintf(name, sizeof(name), "sfft_%s_n%d_xy%d_%s", mode_name<T>(mode, sign), p->n[0],
+             (int)(N1 / R), sizeof(T) == 4 ? "f32" : "f64");
+    return prof_launch(p, name, 2.0 * N0 * N1 * Nh * sizeof(C), launch);
+  }
+
   // ---------------------------------------------------------- public paths
   static int r2c(accfft_amd_plan* p, const void* in, void* out, unsigned xyz) {
     const int64_t Nh = p->n[2] / 2 + 1;
     void* o = out;
     int st;
+    if ((xyz & 7) == 7 && two(p)) {
+      if ((st = two_zy(p, -1, in, out))) return st;
+      return two_xy(p, M_C2C, -1, out, out);
+    }
     if ((xyz & 6) == 6 && yfused(p) && !p->inplace) {
       if ((st = zy_fwd(p, in, out))) return st;
       return (xyz & 1) ? x_c2c(p, out, out, Nh, -1) : ACCFFT_AMD_OK;
@@ -448,6 +517,11 @@ struct Ops {
     int st;
     if (keep) {
       if ((st = ensure_ws(p, 0, (size_t)N0 * N1 * Nh * sizeof(C)))) return st;
+    }
+    if ((xyz & 7) == 7 && two(p)) {
+      void* mid = keep ? p->ws[0] : in;
+      if ((st = two_xy(p, M_C2C, +1, in, mid))) return st;
+      return two_zy(p, +1, mid, out);
     }
     if (xyz & 1) {
       void* dst = keep ? p->ws[0] : cur;
@@ -980,6 +1054,10 @@ struct Ops {
     int st;
     if ((st = ensure_ws(p, 0, (size_t)N0 * N1 * Nh * sizeof(C)))) return st;
     void* w = p->ws[0];
+    if (two(p)) {
+      if ((st = two_xy(p, M_C2C, +1, G, w))) return st;
+      return two_zy(p, +1, w, x, 1);
+    }
     if ((st = x_c2c(p, G, w, Nh, +1))) return st;
     if ((st = y_c2c(p, w, w, Nh, +1))) return st;
     auto a = zargs(w, x, N0 * N1, Nh, N2);
@@ -989,6 +1067,10 @@ struct Ops {
   static int adjoint_c2r(accfft_amd_plan* p, const void* y, void* G) {
     const int64_t N0 = p->n[0], N1 = p->n[1], N2 = p->n[2], Nh = N2 / 2 + 1;
     int st;
+    if (two(p)) {
+      if ((st = two_zy(p, -1, y, G, 1))) return st;
+      return two_xy(p, M_C2C, -1, G, G);
+    }
     auto a = zargs(y, G, N0 * N1, N2, Nh);
     a.adjw = 1;
     if ((st = run_pass<T>(p, "z", false, M_R2C, -1, a, tab(p, 2)))) return st;
@@ -1032,7 +1114,9 @@ struct Ops {
     const int64_t N0 = p->n[0], N1 = p->n[1], N2 = p->n[2], Nh = N2 / 2 + 1;
     const size_t cb = (size_t)N0 * N1 * Nh * sizeof(C);
     if ((st = ensure_ws(p, 0, cb)) || (st = ensure_ws(p, 1, cb))) return st;
-    if (yfused(p)) {
+    if (two(p)) {
+      if ((st = two_zy(p, -1, A, p->ws[0]))) return st;
+    } else if (yfused(p)) {
       if ((st = zy_fwd(p, A, p->ws[0]))) return st;
     } else {
       if ((st = z_r2c(p, A, p->ws[0], false))) return st;
@@ -1041,6 +1125,11 @@ struct Ops {
     const double scale = 1.0 / ((double)N0 * N1 * N2);
     for (int d = 0; d < 3; ++d) {
       if (!(mask & (1u << d)) || !outs[d]) continue;
+      if (two(p)) {
+        if ((st = two_xy(p, M_MULT, -1, p->ws[0], p->ws[1], SYM_GRAD_X + d, scale))) return st;
+        if ((st = two_zy(p, +1, p->ws[1], outs[d]))) return st;
+        continue;
+      }
       if ((st = x_mult(p, p->ws[0], p->ws[1], Nh, SYM_GRAD_X + d, scale))) return st;
       if (yfused(p)) {
         if ((st = zy_inv(p, p->ws[1], p->ws[1], outs[d]))) return st;
@@ -1064,6 +1153,12 @@ struct Ops {
   static int spectral_in(accfft_amd_plan* p, int sym, void* out, const void* A, void* w) {
     const int64_t N0 = p->n[0], N1 = p->n[1], N2 = p->n[2], Nh = N2 / 2 + 1;
     int st;
+    // (the inverse biharmonic and Poisson symbols have no pass-2 form)
+    if (two(p) && (sym <= SYM_INV_LAPLACE || N1 == p->two)) {
+      if ((st = two_zy(p, -1, A, w))) return st;
+      if ((st = two_xy(p, M_MULT, -1, w, w, sym, 1.0 / ((double)N0 * N1 * N2)))) return st;
+      return two_zy(p, +1, w, out);
+    }
     if (yfused(p)) {
       if ((st = zy_fwd(p, A, w))) return st;
       if ((st = x_mult(p, w, w, Nh, sym, 1.0 / ((double)N0 * N1 * N2)))) return st;
@@ -1123,6 +1218,7 @@ struct Ops {
       int64_t in_elems, out_elems;
     };
     std::vector<Pass> passes;
+    if (two(p)) return ACCFFT_AMD_OK;  // its passes have one configuration
     if (p->kind == 1 || p->kind == 2) {
       const int64_t L = p->kind == 1 ? Nh : N2, e = N0 * N1 * L;
       if (!yfused(p)) passes.push_back({1, 1, y_args(p, nullptr, nullptr, L), e, 0});

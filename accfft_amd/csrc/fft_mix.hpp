@@ -413,8 +413,11 @@ struct MixSym {
   double scale;
   bool on_k;  // grad: along the varying axis
   template <typename T>
-  __device__ __forceinline__ MixSym(const FftArgs<T>& a, int64_t col) {
-    const int64_t u = col / a.Ch, Z = col - u * a.Ch;
+  __device__ __forceinline__ MixSym(const FftArgs<T>& a, int64_t col)
+      : MixSym(a, (long)(col / a.Ch), (long)(col % a.Ch)) {}
+  // u: wavenumber index of the other full axis, Z: along z
+  template <typename T>
+  __device__ __forceinline__ MixSym(const FftArgs<T>& a, long u, long Z) {
     const long Nu = a.maxis == 0 ? a.N1 : a.N0;
     scale = a.scale;
     on_k = a.sym == (a.maxis == 0 ? SYM_GRAD_X : SYM_GRAD_Y);

@@ -1,0 +1,33 @@
+// fft_two_launch.hpp -- when a plan takes the two-pass kernels (fft_two.hpp)
+// and how they are launched (fft_two.hip).
+#pragma once
+#include "fft_kernels.hpp"
+
+namespace afft {
+
+inline bool two_pow2(int n, int lo, int hi) { return n >= lo && n <= hi && (n & (n - 1)) == 0; }
+// R of N1 = R M, the rows pass 1 transforms at once (0: no two-pass form).
+// M = 1 leaves pass 2 the plain x pass, which takes any length.
+inline int two_rows(const int* n) {
+  if (!two_pow2(n[2], 32, 512) || !two_pow2(n[1], 32, 512)) return 0;
+  const int r = n[1] == 32 ? 32 : 64;
+  if (n[1] > r && !two_pow2(n[0], 64, 512)) return 0;
+  return r;
+}
+
+// Pass 1 of `a.nlines` = planes x M blocks; sign < 0 r2c, > 0 c2r.
+template <typename T>
+hipError_t launch_two_zy(int sign, int nz, int r, const FftArgs<T>& a, const cpx<T>* twy, hipStream_t st);
+// Pass 2, M_C2C (either sign) or M_MULT.
+template <typename T>
+hipError_t launch_two_xy(int mode, int sign, int n0, int m, const FftArgs<T>& a, hipStream_t st);
+#define AFFT_TWO_DECL(T)                                                                          \
+  template <>                                                                                     \
+  hipError_t launch_two_zy<T>(int, int, int, const FftArgs<T>&, const cpx<T>*, hipStream_t);      \
+  template <>                                                                                     \
+  hipError_t launch_two_xy<T>(int, int, int, int, const FftArgs<T>&, hipStream_t);
+AFFT_TWO_DECL(float)
+AFFT_TWO_DECL(double)
+#undef AFFT_TWO_DECL
+
+}  // namespace afft

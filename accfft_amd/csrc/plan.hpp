@@ -16,6 +16,7 @@
 #include "../../include/accfft_amd.h"
 #include "fft_launch.hpp"
 #include "fft_mix.hpp"
+#include "fft_two_launch.hpp"
 
 struct accfft_amd_plan {
   int n[3] = {0, 0, 0};
@@ -53,6 +54,9 @@ struct accfft_amd_plan {
   // level (set at plan creation when the tables exist; tuning choice -3 on
   // the y axis turns it off, -1 restores it)
   bool yfuse = false;
+  // 1 x 1 out-of-place r2c plans with a two-pass form (fft_two.hpp): R of
+  // N1 = R M, 0 for none; off while a tuning choice is set on the x or y axis
+  int two = 0;
   std::vector<void*> dev_mem;  // table allocations
   // 0, 1: spectra of the operators, adjoints and slab plans (and 2 of the
   // pencil plans); 2, 3: the ping-pong buffers of lines longer than one LDS
