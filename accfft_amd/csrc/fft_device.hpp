@@ -114,36 +114,50 @@ __device__ __forceinline__ void dft8(cpx<T>* v) {
   v[7] = csub(e[3], o3);
 }
 
-// 16 = 2 x 8 (decimation in time)
-template <typename T, int SIGN>
-__device__ __forceinline__ void dft16(cpx<T>* v) {
-  const T c1 = (T)0.92387953251128675613;  // cos(pi/8)
-  const T s1 = (T)0.38268343236508977173;  // sin(pi/8)
-  const T c2 = (T)0.70710678118654752440;
-  cpx<T> e[8], o[8];
-#pragma unroll
-  for (int r = 0; r < 8; ++r) {
-    e[r] = v[2 * r];
-    o[r] = v[2 * r + 1];
+// v exp(SIGN 2 pi i m / 32), m a constant after unrolling: quarter turns cost
+// no arithmetic, odd eighths two products of a sum.
+template <int SIGN, typename T>
+__device__ __forceinline__ cpx<T> rot32(cpx<T> v, int m) {
+  // cos(pi k / 16), k = 0 ... 8
+  const T c[9] = {(T)1, (T)0.98078528040323044913, (T)0.92387953251128675613,
+                  (T)0.83146961230254523708, (T)0.70710678118654752440,
+                  (T)0.55557023301960222474, (T)0.38268343236508977173,
+                  (T)0.19509032201612826785, (T)0};
+  m &= 31;
+  const int q = m >> 3, e = m & 7;  // quarter turns, then e / 32 of a turn
+  if (e == 4) v = {c[4] * (v.x - SIGN * v.y), c[4] * (v.y + SIGN * v.x)};
+  else if (e != 0) {
+    const T wr = c[e], wi = SIGN * c[8 - e];
+    v = {v.x * wr - v.y * wi, v.x * wi + v.y * wr};
   }
-  dft8<T, SIGN>(e);
-  dft8<T, SIGN>(o);
-  // W16^k = cos(pi k/8) + SIGN*i*sin(pi k/8)
-  const T cw[8] = {(T)1, c1, c2, s1, (T)0, -s1, -c2, -c1};
-  const T sw[8] = {(T)0, s1, c2, c1, (T)1, c1, c2, s1};
+  return q == 0 ? v : q == 1 ? mul_si<SIGN>(v) : q == 2 ? cpx<T>{-v.x, -v.y} : mul_si<-SIGN>(v);
+}
+
+// 16 = 4 x 4 and 32 = 8 x 4 (n = B n1 + n2, k = k1 + 4 k2, n1, k1 < 4): one
+// level of rotations between the two (16 as 2 x 8, which has two, is less
+// accurate and takes more products).
+template <typename T, int B, int SIGN>
+__device__ __forceinline__ void dft4xB(cpx<T>* v) {
+  cpx<T> y[4][B];
 #pragma unroll
-  for (int k = 0; k < 8; ++k) {
-    cpx<T> t;
-    if (k == 0) t = o[0];
-    else if (k == 4) t = mul_si<SIGN>(o[4]);
-    else {
-      const T wr = cw[k], wi = SIGN * sw[k];
-      t = {o[k].x * wr - o[k].y * wi, o[k].x * wi + o[k].y * wr};
-    }
-    v[k] = cadd(e[k], t);
-    v[k + 8] = csub(e[k], t);
+  for (int n2 = 0; n2 < B; ++n2) {
+    cpx<T> t[4] = {v[n2], v[B + n2], v[2 * B + n2], v[3 * B + n2]};
+    dft4<T, SIGN>(t);
+#pragma unroll
+    for (int k1 = 0; k1 < 4; ++k1) y[k1][n2] = rot32<SIGN>(t[k1], n2 * k1 * (8 / B));
+  }
+#pragma unroll
+  for (int k1 = 0; k1 < 4; ++k1) {
+    if constexpr (B == 4) dft4<T, SIGN>(y[k1]);
+    else dft8<T, SIGN>(y[k1]);
+#pragma unroll
+    for (int k2 = 0; k2 < B; ++k2) v[k1 + 4 * k2] = y[k1][k2];
   }
 }
+template <typename T, int SIGN>
+__device__ __forceinline__ void dft16(cpx<T>* v) { dft4xB<T, 4, SIGN>(v); }
+template <typename T, int SIGN>
+__device__ __forceinline__ void dft32(cpx<T>* v) { dft4xB<T, 8, SIGN>(v); }
 
 // Odd prime R in {3, 5, 7, 11, 13} by the symmetric pair form:
 //   X[q]   = v0 + sum_r a_r cos(2 pi r q/R) + SIGN*i sum_r b_r sin(2 pi r q/R)

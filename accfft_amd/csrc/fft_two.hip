@@ -33,13 +33,14 @@ hipError_t launch_two_zy<AFFT_T>(int sign, int nz, int r, const FftArgs<AFFT_T>&
 template <>
 hipError_t launch_two_xy<AFFT_T>(int mode, int sign, int n0, int m, const FftArgs<AFFT_T>& a,
                                  hipStream_t st) {
-  const unsigned flip = sign > 0 ? 0x80000000u : 0u;
 #define AFFT_XY(NN, MM)                                                                           \
   if (n0 == NN && m == MM) {                                                                      \
-    using CF = XYCfg<AFFT_T, NN, MM>;                                                             \
-    const dim3 g((unsigned)((a.nlines + CF::W - 1) / CF::W)), b(CF::TPB);                         \
-    if (mode == M_C2C) hipLaunchKernelGGL((two_xy_kernel<AFFT_T, NN, MM, M_C2C>), g, b, 0, st, a, flip); \
-    else if (mode == M_MULT) hipLaunchKernelGGL((two_xy_kernel<AFFT_T, NN, MM, M_MULT>), g, b, 0, st, a, flip); \
+    using CF = XYCfg<AFFT_T, NN, MM, M_C2C>;                                                      \
+    using CM = XYCfg<AFFT_T, NN, MM, M_MULT>;                                                     \
+    const dim3 g((unsigned)((a.nlines + CF::W - 1) / CF::W)), b(mode == M_C2C ? CF::TPB : CM::TPB); \
+    if (mode == M_C2C && sign < 0) hipLaunchKernelGGL((two_xy_kernel<AFFT_T, NN, MM, M_C2C, -1>), g, b, 0, st, a); \
+    else if (mode == M_C2C) hipLaunchKernelGGL((two_xy_kernel<AFFT_T, NN, MM, M_C2C, +1>), g, b, 0, st, a); \
+    else if (mode == M_MULT) hipLaunchKernelGGL((two_xy_kernel<AFFT_T, NN, MM, M_MULT, -1>), g, b, 0, st, a); \
     else return hipErrorNotSupported;                                                             \
     return hipGetLastError();                                                                     \
   }

@@ -18,38 +18,15 @@
 
 namespace afft {
 
-// 32 = 2 x 16 (decimation in time)
-template <typename T, int SIGN>
-__device__ __forceinline__ void dft32(cpx<T>* v) {
-  cpx<T> e[16], o[16];
-#pragma unroll
-  for (int r = 0; r < 16; ++r) {
-    e[r] = v[2 * r];
-    o[r] = v[2 * r + 1];
-  }
-  dft16<T, SIGN>(e);
-  dft16<T, SIGN>(o);
-  // cos / sin of pi k / 16
-  const T cw[16] = {(T)1, (T)0.98078528040323044913, (T)0.92387953251128675613,
-                    (T)0.83146961230254523708, (T)0.70710678118654752440,
-                    (T)0.55557023301960222474, (T)0.38268343236508977173,
-                    (T)0.19509032201612826785, (T)0, (T)-0.19509032201612826785,
-                    (T)-0.38268343236508977173, (T)-0.55557023301960222474,
-                    (T)-0.70710678118654752440, (T)-0.83146961230254523708,
-                    (T)-0.92387953251128675613, (T)-0.98078528040323044913};
-#pragma unroll
-  for (int k = 0; k < 16; ++k) {
-    cpx<T> t;
-    if (k == 0) t = o[0];
-    else if (k == 8) t = mul_si<SIGN>(o[8]);
-    else {
-      const T wr = cw[k], wi = SIGN * cw[k < 8 ? 8 - k : k - 8];  // sin(pi k/16) = cos(pi (8-k)/16)
-      t = {o[k].x * wr - o[k].y * wi, o[k].x * wi + o[k].y * wr};
-    }
-    v[k] = cadd(e[k], t);
-    v[k + 16] = csub(e[k], t);
-  }
+// Element at 32-bit byte offset `off` of a uniform base: the base stays in
+// scalar registers (scalar arithmetic for the row steps) and a thread keeps
+// one offset register for all of its loads.  The grids of this file are at
+// most 512^3 FP64 spectra, 2.2 GB.
+template <typename V, typename B>
+__device__ __forceinline__ gptr<V> at_off(B* base, uint32_t off) {
+  return (gptr<V>)((gptr<typename std::conditional<std::is_const<B>::value, const char, char>::type>)base + off);
 }
+
 template <typename T, int R, int SIGN>
 __device__ __forceinline__ void pdft(cpx<T>* v) {
   if constexpr (R == 1) return;
@@ -65,22 +42,27 @@ __device__ __forceinline__ void pdft(cpx<T>* v) {
 // L = M W values, the n2 groups rotated by XOR with x / R0: the first stage
 // writes M consecutive j = x / R0 from one wavefront, which would otherwise
 // fall on the same W banks.
-template <typename T, int N0, int M>
+template <typename T, int N0, int M, int MODE>
 struct XYCfg {
-  // elements a thread: 64 registers of data
-  static constexpr int E = sizeof(T) == 4 ? 32 : 16;
+  // 64-byte row segments for tiles of 1024 rows and more (FP64: 128 bytes
+  // below 4096 rows), 128 bytes for shorter ones
+  static constexpr int W = sizeof(T) == 4 ? (M * N0 >= 1024 ? 8 : 16) : (M * N0 >= 4096 ? 4 : 8);
+  // elements a thread: 64 registers of data; the FP32 multiply of short
+  // tiles half of that (it needs registers for the symbol and the way back:
+  // 128^3 16.3 -> 13.3 us, from 1024 rows 43 us with 32, 45 with 16)
+  static constexpr int E = sizeof(T) == 8 || (MODE == M_MULT && M * N0 < 1024) ? 16 : 32;
+  // waves per SIMD of the multiply: three leave it 168 registers, with four
+  // it spills 30 to 70 (256^3 FP32 52 against 42 us)
+  static constexpr int MULT_WAVES = 3;
   static constexpr int R0 = E / M;
   static constexpr int NR = N0 / R0;  // left for R1 R2
   static constexpr int R2 = NR <= 16 ? 1 : NR <= 64 ? 8 : 16;
   static constexpr int R1 = NR / R2;
-  // 64-byte row segments for tiles of 1024 rows and more (FP64: 128 bytes
-  // below 4096 rows), 128 bytes for shorter ones
-  static constexpr int W = sizeof(T) == 4 ? (M * N0 >= 1024 ? 8 : 16) : (M * N0 >= 4096 ? 4 : 8);
   static constexpr int TPB = NR * W;
 };
-template <typename T, int N0, int M>
+template <typename T, int N0, int M, int MODE>
 struct XYTile {
-  using CF = XYCfg<T, N0, M>;
+  using CF = XYCfg<T, N0, M, MODE>;
   static constexpr int W = CF::W, TPB = CF::TPB, R0 = CF::R0, R1 = CF::R1, R2 = CF::R2, L = M * W;
   static constexpr int NB1 = N0 / R1, P1 = NB1 * L / TPB, NB2 = N0 / R2, P2 = NB2 * L / TPB;
   static constexpr int NS1 = R0, NS2 = R0 * R1;
@@ -172,16 +154,16 @@ struct XYTile {
 #pragma unroll
     for (int i = 0; i < M; ++i) pdft<T, R0, SIGN>(v[i]);
   }
-  // stage 1 or 2 on the registers: forward twiddles then DFTs, inverse DFTs
-  // then conjugate twiddles
-  template <int PER, int R, int NS, int SIGN>
+  // stage 1 or 2 on the registers: twiddles then DFTs, or (BACK: a stage
+  // undone) DFTs then twiddles
+  template <int PER, int R, int NS, int SIGN, bool BACK>
   static __device__ __forceinline__ void stage(cpx<T> (&x)[PER][R], int t, const cpx<T>* tw) {
 #pragma unroll
     for (int i = 0; i < PER; ++i) {
       const int j = (t + i * TPB) / L;
-      if constexpr (SIGN < 0) twiddle<R, NS, SIGN>(x[i], j, tw);
+      if constexpr (!BACK) twiddle<R, NS, SIGN>(x[i], j, tw);
       pdft<T, R, SIGN>(x[i]);
-      if constexpr (SIGN > 0) twiddle<R, NS, SIGN>(x[i], j, tw);
+      if constexpr (BACK) twiddle<R, NS, SIGN>(x[i], j, tw);
     }
   }
 };
@@ -223,86 +205,70 @@ struct TwoSym {
 
 // In place or out of place over [N0][N1][Nh]: a.Sin / a.Sout the x strides,
 // a.Din / a.Dout the n2 strides (R Nh), a.nlines = R Nh columns, a.tw the
-// full table of N0.  M_C2C: flip as in mix_s_kernel.  M_MULT: forward, the
+// full table of N0.  M_C2C: transforms of sign SIGN.  M_MULT: forward, the
 // symbol a.sym (a.Ch = Nh, a.C = R), inverse, the inverse running the
 // forward stages backwards.
-template <typename T, int N0, int M, int MODE>
-__global__ void __launch_bounds__((XYCfg<T, N0, M>::TPB), 4)
-    two_xy_kernel(FftArgs<T> a, unsigned flip) {
-  using K = XYTile<T, N0, M>;
+template <typename T, int N0, int M, int MODE, int SIGN>
+__global__ void __launch_bounds__((XYCfg<T, N0, M, MODE>::TPB), (MODE == M_MULT ? XYCfg<T, N0, M, MODE>::MULT_WAVES : 4))
+    two_xy_kernel(FftArgs<T> a) {
+  using K = XYTile<T, N0, M, MODE>;
   constexpr int W = K::W, TPB = K::TPB, R0 = K::R0, R1 = K::R1, R2 = K::R2, L = K::L;
+  static_assert(MODE == M_C2C || SIGN < 0, "M_MULT starts forward");
   __shared__ T buf[N0 * L];
   __shared__ cpx<T> tw[K::TWN];
   const int t = threadIdx.x;
   int64_t tile = xcd_tile(blockIdx.x, gridDim.x, (unsigned)a.xgroup);
   if (a.reverse) tile = (int64_t)gridDim.x - 1 - tile;
   const int64_t col0 = tile * W;
-  // first-stage registers: column c0, x = t / W + r N0 / R0, all n2
-  const int64_t c0 = col0 + t % W;
-  const bool ok0 = c0 < a.nlines;
+  const int cols = a.nlines - col0 < W ? (int)(a.nlines - col0) : W;  // of this tile
+  // first-stage registers: column t % W (clamped: a column past the last
+  // one repeats it and is not stored), x = t / W + r N0 / R0, all n2
   typename K::V0 v;
   {
-    const int64_t step = (int64_t)(N0 / R0) * a.Sin;
-    gptr<const cpx<T>> p = to_global(reinterpret_cast<const cpx<T>*>(a.in) + c0 + (int64_t)(t / W) * a.Sin);
+    const int c = t % W < cols ? t % W : cols - 1;
+    const uint32_t off = (uint32_t)((c + (t / W) * a.Sin) * sizeof(cpx<T>));
+    const cpx<T>* src = reinterpret_cast<const cpx<T>*>(a.in) + col0;
 #pragma unroll
-    for (int r = 0; r < R0; ++r) {
-      gptr<const cpx<T>> q = p;
+    for (int r = 0; r < R0; ++r)
 #pragma unroll
-      for (int i = 0; i < M; ++i) {
-        v[i][r] = ok0 ? ld_global(q) : cpx<T>{(T)0, (T)0};
-        q += a.Din;
-        asm volatile("" : "+v"(q));
-      }
-      p += step;
-      asm volatile("" : "+v"(p));
-    }
+      for (int i = 0; i < M; ++i)
+        v[i][r] = ld_global(at_off<const cpx<T>>(src + r * (N0 / R0) * a.Sin + i * a.Din, off));
   }
   K::stage_tw(tw, a.tw, t);
-  if constexpr (MODE == M_C2C) {
-#pragma unroll
-    for (int i = 0; i < M; ++i)
-#pragma unroll
-      for (int r = 0; r < R0; ++r) v[i][r] = conj_if(v[i][r], flip);
-  }
   auto w0 = [&](int i, int r) { return K::w0(t, i, r); };
   auto r1 = [&](int i, int r) { return K::r1(t, i, r); };
   auto w1 = [&](int i, int r) { return K::w1(t, i, r); };
   auto r2 = [&](int i, int r) { return K::r2(t, i, r); };
-  K::template first<-1>(v);
+  K::template first<SIGN>(v);
   typename K::V1 x;
   K::exchange(v, x, buf, false, w0, r1);
-  K::template stage<K::P1, R1, K::NS1, -1>(x, t, tw);
+  K::template stage<K::P1, R1, K::NS1, SIGN, false>(x, t, tw);
   // the last stage's outputs: row x = j + r N0 / R, row n2 -> k2 and column
   // of this thread
   const int line = t % L;
-  const int64_t col = col0 + line % W;
   if constexpr (MODE == M_C2C) {
     auto store = [&](auto& o, auto per, auto rad) {
       constexpr int PER = decltype(per)::value, R = decltype(rad)::value;
-      if (col >= a.nlines) return;
-      cpx<T>* dst = reinterpret_cast<cpx<T>*>(a.out) + col + (int64_t)(line / W) * a.Dout;
-      const int64_t step = (int64_t)(N0 / R) * a.Sout;
+      if (line % W >= cols) return;
+      cpx<T>* dst = reinterpret_cast<cpx<T>*>(a.out) + col0;
+      const uint32_t off = (uint32_t)((line % W + (line / W) * a.Dout + (t / L) * a.Sout) * sizeof(cpx<T>));
 #pragma unroll
-      for (int i = 0; i < PER; ++i) {
-        gptr<cpx<T>> p = to_global(dst + (int64_t)((t + i * TPB) / L) * a.Sout);
+      for (int i = 0; i < PER; ++i)
 #pragma unroll
-        for (int r = 0; r < R; ++r) {
-          *p = conj_if(o[i][r], flip);
-          p += step;
-          asm volatile("" : "+v"(p));
-        }
-      }
+        for (int r = 0; r < R; ++r)
+          *at_off<cpx<T>>(dst + (i * (TPB / L) + r * (N0 / R)) * a.Sout, off) = o[i][r];
     };
     if constexpr (R2 > 1) {
       typename K::V2 o;
       K::exchange(x, o, buf, true, w1, r2);
-      K::template stage<K::P2, R2, K::NS2, -1>(o, t, tw + K::OFF2);
+      K::template stage<K::P2, R2, K::NS2, SIGN, false>(o, t, tw + K::OFF2);
       store(o, std::integral_constant<int, K::P2>{}, std::integral_constant<int, R2>{});
     } else {
       store(x, std::integral_constant<int, K::P1>{}, std::integral_constant<int, R1>{});
     }
     return;
   } else {
+    const int64_t col = col0 + line % W;
     const int64_t k1 = col / a.Ch;
     const TwoSym<T> sym(a, (int)(k1 + a.C * (line / W)), (int)(col - k1 * a.Ch));
     auto symbol = [&](auto& o, auto per, auto rad) {
@@ -332,33 +298,25 @@ __global__ void __launch_bounds__((XYCfg<T, N0, M>::TPB), 4)
     if constexpr (R2 > 1) {
       typename K::V2 o;
       K::exchange(x, o, buf, true, w1, r2);
-      K::template stage<K::P2, R2, K::NS2, -1>(o, t, tw + K::OFF2);
+      K::template stage<K::P2, R2, K::NS2, -1, false>(o, t, tw + K::OFF2);
       symbol(o, std::integral_constant<int, K::P2>{}, std::integral_constant<int, R2>{});
-      K::template stage<K::P2, R2, K::NS2, +1>(o, tb, tw + K::OFF2);
+      K::template stage<K::P2, R2, K::NS2, +1, true>(o, tb, tw + K::OFF2);
       // (a thread writes where it alone has read: no barrier)
       K::exchange(o, x, buf, false, br2, bw1);
     } else {
       symbol(x, std::integral_constant<int, K::P1>{}, std::integral_constant<int, R1>{});
     }
-    K::template stage<K::P1, R1, K::NS1, +1>(x, tb, tw);
+    K::template stage<K::P1, R1, K::NS1, +1, true>(x, tb, tw);
     K::exchange(x, v, buf, R2 > 1, br1, bw0);
     K::template first<+1>(v);
-    const int64_t cb = col0 + tb % W;
-    if (cb >= a.nlines) return;
-    const int64_t step = (int64_t)(N0 / R0) * a.Sout;
-    gptr<cpx<T>> p = to_global(reinterpret_cast<cpx<T>*>(a.out) + cb + (int64_t)(tb / W) * a.Sout);
+    if (tb % W >= cols) return;
+    cpx<T>* dst = reinterpret_cast<cpx<T>*>(a.out) + col0;
+    const uint32_t off = (uint32_t)((tb % W + (tb / W) * a.Sout) * sizeof(cpx<T>));
 #pragma unroll
-    for (int r = 0; r < R0; ++r) {
-      gptr<cpx<T>> q = p;
+    for (int r = 0; r < R0; ++r)
 #pragma unroll
-      for (int i = 0; i < M; ++i) {
-        *q = v[i][r];
-        q += a.Dout;
-        asm volatile("" : "+v"(q));
-      }
-      p += step;
-      asm volatile("" : "+v"(p));
-    }
+      for (int i = 0; i < M; ++i)
+        *at_off<cpx<T>>(dst + r * (N0 / R0) * a.Sout + i * a.Dout, off) = v[i][r];
   }
 }
 
@@ -376,19 +334,21 @@ constexpr int two_log(int n) {
   while ((1 << l) < n) ++l;
   return l;
 }
-constexpr TwoSched two_sched(int P, int NZ, int E) {
+// As much of one dimension as fits a butterfly, then the other: few stages
+// with twiddles.  rows_first: the first stage takes whole z rows (lanes along
+// z: the loads of r2c), otherwise the last one does (the stores of c2r).
+constexpr TwoSched two_sched(int P, int NZ, int E, bool rows_first) {
   TwoSched m{0, {}, {}};
   int h = two_log(P), z = two_log(NZ);
   const int e = two_log(E);
   while (h + z > 0) {
-    int bp = (e + 1) / 2 < h ? (e + 1) / 2 : h;
-    int bz = e - bp < z ? e - bp : z;
-    if (bp + bz < e && bp < h) bp = h < e - bz ? h : e - bz;
-    m.bp[m.s] = bp;
-    m.bz[m.s] = bz;
+    int &d0 = rows_first ? h : z, &d1 = rows_first ? z : h;
+    const int b0 = e < d0 ? e : d0, b1 = e - b0 < d1 ? e - b0 : d1;
+    d0 -= b0;
+    d1 -= b1;
+    m.bp[m.s] = rows_first ? b0 : b1;
+    m.bz[m.s] = rows_first ? b1 : b0;
     ++m.s;
-    h -= bp;
-    z -= bz;
   }
   return m;
 }
@@ -400,11 +360,11 @@ struct ZYCfg {
   static constexpr int E = P * NZ / EM >= 256 ? EM : P * NZ / (EM / 2) >= 256 ? EM / 2 : EM / 4;
   static constexpr int TPB = P * NZ / E;
 };
-template <typename T, int P, int NZ>
+template <typename T, int P, int NZ, bool ROWS_FIRST>
 struct ZYTile {
   using CF = ZYCfg<T, P, NZ>;
   static constexpr int E = CF::E, TPB = CF::TPB;
-  static constexpr TwoSched SC = two_sched(P, NZ, E);
+  static constexpr TwoSched SC = two_sched(P, NZ, E, ROWS_FIRST);
   static constexpr int S = SC.s;
   static_assert(TPB >= 64 && TPB <= 1024 && TPB % 64 == 0, "tile shape");
   // LDS: rows of NZ values, five pad values after every 64: a first z stage
@@ -580,14 +540,15 @@ __device__ __forceinline__ cpx<T> cmul2(cpx<T> a, cpx<T> b, cpx<T> c, cpx<T> d) 
 
 // Factors of the split: te[k1] = w^(n2 k1) for the even rows' part of row k1,
 // to[k1] = te[k1] w_R^(k1 mod P) for the odd rows', w = exp(-2 pi i / N1) (one
-// table entry each: one rounding instead of two products in a row).
+// table entry each: one rounding instead of two products in a row), times
+// scale.
 template <typename T, int R, int TPB>
 __device__ __forceinline__ void split_factors(cpx<T>* te, cpx<T>* to, const cpx<T>* __restrict__ twy,
-                                              int n2, int M, int t) {
+                                              int n2, int M, T scale, int t) {
   for (int k = t; k < R; k += TPB) {
     const int e = n2 * k, o = e + M * (k & (R / 2 - 1));
-    te[k] = twy[e];
-    to[k] = twy[o < M * R ? o : o - M * R];
+    te[k] = cscale(twy[e], scale);
+    to[k] = cscale(twy[o < M * R ? o : o - M * R], scale);
   }
 }
 
@@ -604,7 +565,7 @@ template <typename T, int NZ, int R>
 __global__ void __launch_bounds__((ZYCfg<T, R / 2, NZ>::TPB))
     two_zy_r2c_kernel(FftArgs<T> a, const cpx<T>* __restrict__ twy) {
   constexpr int P = R / 2, NH = NZ / 2 + 1;
-  using K = ZYTile<T, P, NZ>;
+  using K = ZYTile<T, P, NZ, true>;
   constexpr int TPB = K::TPB, I = P * (NZ / 2) / TPB;
   __shared__ T buf[P * K::ZP];
   __shared__ cpx<T> twz[K::TWZ], twp[K::TWP], te[R], to[R];
@@ -620,23 +581,19 @@ __global__ void __launch_bounds__((ZYCfg<T, R / 2, NZ>::TPB))
     for (int i = 0; i < S0::PER; ++i) {
       int pj, zj;
       S0::map(t, i, pj, zj);
-      gptr<const T> p = to_global(src + (int64_t)(2 * pj) * row + zj);
+      const uint32_t off = (uint32_t)((2 * pj * row + zj) * sizeof(T));
 #pragma unroll
-      for (int r = 0; r < S0::RP; ++r) {
-        gptr<const T> p1 = p + row;
+      for (int r = 0; r < S0::RP; ++r)
 #pragma unroll
         for (int q = 0; q < S0::RZ; ++q) {
-          v[i][r][q].x = p[q * S0::NBZ];
-          v[i][r][q].y = p1[q * S0::NBZ];
+          v[i][r][q].x = *at_off<const T>(src + 2 * r * S0::NBP * row + q * S0::NBZ, off);
+          v[i][r][q].y = *at_off<const T>(src + (2 * r * S0::NBP + 1) * row + q * S0::NBZ, off);
         }
-        p += 2 * S0::NBP * row;
-        asm volatile("" : "+v"(p));
-      }
     }
   }
   K::template stage_tw<true>(twz, a.tw, 1, t);
   K::template stage_tw<false>(twp, twy, 2 * (int)M, t);  // roots of P = N1 / (2 M)
-  split_factors<T, R, TPB>(te, to, twy, (int)n2, (int)M, t);
+  split_factors<T, R, TPB>(te, to, twy, (int)n2, (int)M, (T)0.5, t);
   typename K::template Regs<K::S - 1> o;
   K::template run<0, -1>(v, o, buf, t, false, twp, twz);
   // U in natural order through the LDS (each thread writes where it alone
@@ -669,15 +626,16 @@ __global__ void __launch_bounds__((ZYCfg<T, R / 2, NZ>::TPB))
   __syncthreads();
   grab(ay, by);
   cpx<T>* dst = reinterpret_cast<cpx<T>*>(a.out) + x * a.Dout + n2 * R * a.odist;
-  const T h = (T)0.5;
 #pragma unroll
   for (int i = 0; i <= I; ++i) {
     if (i == I && t >= P) break;
     int q, k;
     item(i, q, k);
-    const T s = (a.adjw && k != 0 && k != NZ / 2) ? (T)1 : h;
-    const cpx<T> e = {s * (ax[i] + bx[i]), s * (ay[i] - by[i])};
-    const cpx<T> d = {s * (ay[i] + by[i]), s * (bx[i] - ax[i])};
+    cpx<T> e = {ax[i] + bx[i], ay[i] - by[i]}, d = {ay[i] + by[i], bx[i] - ax[i]};
+    if (a.adjw && k != 0 && k != NZ / 2) {  // (the factors carry the 1/2)
+      e = cscale(e, (T)2);
+      d = cscale(d, (T)2);
+    }
     cpx<T>* p = dst + q * a.odist + k;
     p[0] = cmul2<T, 1, false>(e, te[q], d, to[q]);
     p[P * a.odist] = cmul2<T, -1, false>(e, te[q + P], d, to[q + P]);
@@ -693,7 +651,7 @@ template <typename T, int NZ, int R>
 __global__ void __launch_bounds__((ZYCfg<T, R / 2, NZ>::TPB))
     two_zy_c2r_kernel(FftArgs<T> a, const cpx<T>* __restrict__ twy) {
   constexpr int P = R / 2;
-  using K = ZYTile<T, P, NZ>;
+  using K = ZYTile<T, P, NZ, false>;
   constexpr int TPB = K::TPB, I = P * (NZ / 2) / TPB;
   __shared__ T buf[P * K::ZP];
   __shared__ cpx<T> twz[K::TWZ], twp[K::TWP], te[R], to[R], edge[2][2][P];
@@ -718,9 +676,8 @@ __global__ void __launch_bounds__((ZYCfg<T, R / 2, NZ>::TPB))
   }
   K::template stage_tw<true>(twz, a.tw, 1, t);
   K::template stage_tw<false>(twp, twy, 2 * (int)M, t);
-  split_factors<T, R, TPB>(te, to, twy, (int)n2, (int)M, t);
+  split_factors<T, R, TPB>(te, to, twy, (int)n2, (int)M, (T)1, t);
   __syncthreads();
-  const T s = a.adjw ? (T)0.5 : (T)1;
 #pragma unroll
   for (int i = 0; i < I; ++i) {
     const int b = t + i * TPB, k = b % (NZ / 2), q = b / (NZ / 2);
@@ -730,8 +687,15 @@ __global__ void __launch_bounds__((ZYCfg<T, R / 2, NZ>::TPB))
       edge[0][0][q] = e;
       edge[0][1][q] = d;
     }
-    y0[i] = {s * (e.x - d.y), s * (e.y + d.x)};
-    y1[i] = {s * (e.x + d.y), s * (d.x - e.y)};
+    y0[i] = {e.x - d.y, e.y + d.x};
+    y1[i] = {e.x + d.y, d.x - e.y};
+  }
+  if (a.adjw) {
+#pragma unroll
+    for (int i = 0; i < I; ++i) {
+      y0[i] = cscale(y0[i], (T)0.5);
+      y1[i] = cscale(y1[i], (T)0.5);
+    }
   }
   if (t < P) {
     edge[1][0][t] = cmul2<T, 1, true>(z0, te[t], z1, te[t + P]);
@@ -777,18 +741,14 @@ __global__ void __launch_bounds__((ZYCfg<T, R / 2, NZ>::TPB))
   for (int i = 0; i < SL::PER; ++i) {
     int pj, zj;
     SL::map(t, i, pj, zj);
-    gptr<T> p = to_global(dst + (int64_t)(2 * pj) * row + zj);
+    const uint32_t off = (uint32_t)((2 * pj * row + zj) * sizeof(T));
 #pragma unroll
-    for (int r = 0; r < SL::RP; ++r) {
-      gptr<T> p1 = p + row;
+    for (int r = 0; r < SL::RP; ++r)
 #pragma unroll
       for (int q = 0; q < SL::RZ; ++q) {
-        p[q * SL::NBZ] = o[i][r][q].x;
-        p1[q * SL::NBZ] = o[i][r][q].y;
+        *at_off<T>(dst + 2 * r * SL::NBP * row + q * SL::NBZ, off) = o[i][r][q].x;
+        *at_off<T>(dst + (2 * r * SL::NBP + 1) * row + q * SL::NBZ, off) = o[i][r][q].y;
       }
-      p += 2 * SL::NBP * row;
-      asm volatile("" : "+v"(p));
-    }
   }
 }
 
