@@ -146,9 +146,26 @@ def _check(status: int, what: str) -> None:
         raise AccfftError(f"{what}: {msg} (status {status})", status)
 
 
+_raw_stream = None
+
+
 def _stream():
-    import torch
-    return ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+    """torch's current stream on the current device, as an address.  Read
+    through torch's raw accessors: the Stream object that
+    torch.cuda.current_stream() builds takes 3 us, a quarter of a small
+    transform's call (64^3 FP64 round trip, two calls: 24.8 -> 21.7 us)."""
+    global _raw_stream
+    if _raw_stream is None:
+        import torch
+        first = torch.cuda.current_stream().cuda_stream  # initialises the device
+        get = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+        dev = getattr(torch._C, "_cuda_getDevice", None)
+        if get is None or dev is None:
+            _raw_stream = lambda: torch.cuda.current_stream().cuda_stream
+        else:
+            _raw_stream = lambda: get(dev())
+        return first
+    return _raw_stream()
 
 
 def _ptr(t) -> Optional[int]:
