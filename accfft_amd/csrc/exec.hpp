@@ -421,7 +421,7 @@ struct Ops {
   }
 
   // ---------------------------------------------------------- two passes
-  // 1 x 1 r2c plans on power-of-two grids (fft_two.hpp).  A tuning choice on
+  // 1 x 1 r2c and c2c plans on power-of-two grids (fft_two.hpp).  A tuning choice on
   // the x or y axis, or the separate z and y passes (choice -3), takes the
   // plan back to one pass per axis.
   static bool two(const accfft_amd_plan* p) {
@@ -451,10 +451,32 @@ struct Ops {
              sizeof(T) == 4 ? "f32" : "f64");
     return prof_launch(p, name, (double)(N0 * N1) * (N2 * sizeof(T) + Nh * sizeof(C)), launch);
   }
-  // pass 2 over the half spectrum
+  // pass 1 of a c2c transform, in != out
+  static int two_zy_c2c(accfft_amd_plan* p, int sign, const void* in, void* out) {
+    const int64_t N0 = p->n[0], N1 = p->n[1], N2 = p->n[2], M = N1 / p->two;
+    FftArgs<T> a{};
+    a.in = in;
+    a.out = out;
+    a.idist = a.odist = N2;
+    a.Din = a.Dout = N1 * N2;
+    a.C = M;
+    a.nlines = N0 * M;
+    a.tw = tab(p, 2).tw_full;
+    a.xgroup = xcd_group_z();
+    auto launch = [&]() {
+      return launch_two_zy_c2c<T>(sign, p->n[2], p->two, a, tab(p, 1).tw_full, p->stream);
+    };
+    if (!p->prof) return status_of(launch());
+    char name[64];
+    snprintf(name, sizeof(name), "zyfft_%s_n%d_zy%d_%s", mode_name<T>(M_C2C, sign), p->n[2], p->two,
+             sizeof(T) == 4 ? "f32" : "f64");
+    return prof_launch(p, name, 2.0 * N0 * N1 * N2 * sizeof(C), launch);
+  }
+  // pass 2 over the half (c2c: the whole) spectrum
   static int two_xy(accfft_amd_plan* p, int mode, int sign, const void* in, void* out, int sym = 0,
                     double scale = 0) {
-    const int64_t N0 = p->n[0], N1 = p->n[1], Nh = p->n[2] / 2 + 1, R = p->two;
+    const int64_t N0 = p->n[0], N1 = p->n[1], R = p->two;
+    const int64_t Nh = p->kind == 2 ? p->n[2] : p->n[2] / 2 + 1;
     if (N1 == R) {
       if (mode == M_MULT) return x_mult(p, in, out, Nh, sym, scale);
       return x_c2c(p, in, out, Nh, sign);
@@ -542,6 +564,10 @@ struct Ops {
   static int c2c(accfft_amd_plan* p, int dir, void* in, void* out, unsigned xyz) {
     const int64_t N0 = p->n[0], N1 = p->n[1], N2 = p->n[2];
     int st;
+    if ((xyz & 7) == 7 && two(p) && in != out) {  // (the inverse leaves its input alone)
+      if ((st = two_zy_c2c(p, dir, in, out))) return st;
+      return two_xy(p, M_C2C, dir, out, out);
+    }
     if (dir < 0) {
       void* o = out;
       if (xyz & 4) {

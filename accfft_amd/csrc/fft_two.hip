@@ -31,6 +31,32 @@ hipError_t launch_two_zy<AFFT_T>(int sign, int nz, int r, const FftArgs<AFFT_T>&
 }
 
 template <>
+hipError_t launch_two_zy_c2c<AFFT_T>(int sign, int nz, int r, const FftArgs<AFFT_T>& a,
+                                     const cpx<AFFT_T>* twy, hipStream_t st) {
+  const dim3 g((unsigned)a.nlines);
+#define AFFT_ZC(NZ, R)                                                                            \
+  if constexpr (two_c2c_tile<AFFT_T>(NZ, R))                                                      \
+    if (nz == NZ && r == R) {                                                                     \
+      const dim3 b(ZYCfg<AFFT_T, R, NZ>::TPB);                                                    \
+      if (sign < 0) hipLaunchKernelGGL((two_zy_c2c_kernel<AFFT_T, NZ, R, -1>), g, b, 0, st, a, twy); \
+      else hipLaunchKernelGGL((two_zy_c2c_kernel<AFFT_T, NZ, R, +1>), g, b, 0, st, a, twy);       \
+      return hipGetLastError();                                                                   \
+    }
+  AFFT_ZC(32, 32)
+  AFFT_ZC(64, 32)
+  AFFT_ZC(128, 32)
+  AFFT_ZC(256, 32)
+  AFFT_ZC(512, 32)
+  AFFT_ZC(32, 64)
+  AFFT_ZC(64, 64)
+  AFFT_ZC(128, 64)
+  AFFT_ZC(256, 64)
+  AFFT_ZC(512, 64)
+#undef AFFT_ZC
+  return hipErrorNotSupported;
+}
+
+template <>
 hipError_t launch_two_xy<AFFT_T>(int mode, int sign, int n0, int m, const FftArgs<AFFT_T>& a,
                                  hipStream_t st) {
 #define AFFT_XY(NN, MM)                                                                           \
@@ -45,6 +71,7 @@ hipError_t launch_two_xy<AFFT_T>(int mode, int sign, int n0, int m, const FftArg
     return hipGetLastError();                                                                     \
   }
 #define AFFT_XYM(NN) AFFT_XY(NN, 2) AFFT_XY(NN, 4) AFFT_XY(NN, 8)
+  AFFT_XYM(32)
   AFFT_XYM(64)
   AFFT_XYM(128)
   AFFT_XYM(256)

@@ -50,7 +50,9 @@ struct XYCfg {
   // elements a thread: 64 registers of data; the FP32 multiply of short
   // tiles half of that (it needs registers for the symbol and the way back:
   // 128^3 16.3 -> 13.3 us, from 1024 rows 43 us with 32, 45 with 16)
-  static constexpr int E = sizeof(T) == 8 || (MODE == M_MULT && M * N0 < 1024) ? 16 : 32;
+  // (and of 32-point x axes, whose blocks would fall below a wavefront)
+  static constexpr int E = sizeof(T) == 8 ? (N0 * M <= 64 ? 8 : 16)
+                           : N0 <= 32 || (MODE == M_MULT && M * N0 < 1024) ? 16 : 32;
   // waves per SIMD of the multiply: three leave it 168 registers, with four
   // it spills 30 to 70 (256^3 FP32 52 against 42 us)
   static constexpr int MULT_WAVES = 3;
@@ -639,6 +641,58 @@ __global__ void __launch_bounds__((ZYCfg<T, R / 2, NZ>::TPB))
     cpx<T>* p = dst + q * a.odist + k;
     p[0] = cmul2<T, 1, false>(e, te[q], d, to[q]);
     p[P * a.odist] = cmul2<T, -1, false>(e, te[q + P], d, to[q + P]);
+  }
+}
+
+// Pass 1 of a c2c transform, either sign: the complex rows n2 + M n1 -> rows
+// k1 + R n2, transformed along z and over n1 and twiddled for the M-point
+// level.  (The inverse c2c runs the two passes in the same order with the
+// other sign.)  Arguments as above.
+template <typename T, int NZ, int R, int SIGN>
+__global__ void __launch_bounds__((ZYCfg<T, R, NZ>::TPB))
+    two_zy_c2c_kernel(FftArgs<T> a, const cpx<T>* __restrict__ twy) {
+  using K = ZYTile<T, R, NZ, true>;
+  constexpr int TPB = K::TPB;
+  __shared__ T buf[R * K::ZP];
+  __shared__ cpx<T> twz[K::TWZ], twp[K::TWP], te[R];
+  const int t = threadIdx.x;
+  const int64_t blk = xcd_tile(blockIdx.x, gridDim.x, (unsigned)a.xgroup);
+  const int64_t M = a.C, x = blk / M, n2 = blk - x * M;
+  using S0 = typename K::template St<0>;
+  using SL = typename K::Last;
+  typename K::template Regs<0> v;
+  const cpx<T>* src = reinterpret_cast<const cpx<T>*>(a.in) + x * a.Din + n2 * a.idist;
+  const int64_t row = M * a.idist;
+#pragma unroll
+  for (int i = 0; i < S0::PER; ++i) {
+    int pj, zj;
+    S0::map(t, i, pj, zj);
+    const uint32_t off = (uint32_t)((pj * row + zj) * sizeof(cpx<T>));
+#pragma unroll
+    for (int r = 0; r < S0::RP; ++r)
+#pragma unroll
+      for (int q = 0; q < S0::RZ; ++q)
+        v[i][r][q] = ld_global(at_off<const cpx<T>>(src + r * S0::NBP * row + q * S0::NBZ, off));
+  }
+  K::template stage_tw<true>(twz, a.tw, 1, t);
+  K::template stage_tw<false>(twp, twy, (int)M, t);  // roots of R = N1 / M
+  for (int k = t; k < R; k += TPB) te[k] = twy[n2 * k];
+  typename K::template Regs<K::S - 1> o;
+  K::template run<0, SIGN>(v, o, buf, t, false, twp, twz);
+  cpx<T>* dst = reinterpret_cast<cpx<T>*>(a.out) + x * a.Dout + n2 * R * a.odist;
+#pragma unroll
+  for (int i = 0; i < SL::PER; ++i) {
+    int pj, zj;
+    SL::map(t, i, pj, zj);
+    const uint32_t off = (uint32_t)((pj * a.odist + zj) * sizeof(cpx<T>));
+#pragma unroll
+    for (int r = 0; r < SL::RP; ++r) {
+      const cpx<T> w = te[pj + r * SL::NBP];
+#pragma unroll
+      for (int q = 0; q < SL::RZ; ++q)
+        *at_off<cpx<T>>(dst + r * SL::NBP * a.odist + q * SL::NBZ, off) =
+            SIGN < 0 ? cmul(o[i][r][q], w) : cmulc(o[i][r][q], w);
+    }
   }
 }
 

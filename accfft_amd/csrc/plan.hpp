@@ -54,7 +54,7 @@ struct accfft_amd_plan {
   // level (set at plan creation when the tables exist; tuning choice -3 on
   // the y axis turns it off, -1 restores it)
   bool yfuse = false;
-  // 1 x 1 out-of-place r2c plans with a two-pass form (fft_two.hpp): R of
+  // 1 x 1 out-of-place r2c and c2c plans with a two-pass form (fft_two.hpp): R of
   // N1 = R M, 0 for none; off while a tuning choice is set on the x or y axis
   int two = 0;
   std::vector<void*> dev_mem;  // table allocations

@@ -15,7 +15,7 @@ pytestmark = pytest.mark.gpu
 
 SHAPES = ([(3, 32, z) for z in (32, 64, 128, 256, 512)] +
           [(5, 64, z) for z in (32, 64, 128, 256, 512)] +
-          [(x, y, 32) for x in (64, 128, 256, 512) for y in (128, 256, 512)] +
+          [(x, y, 32) for x in (32, 64, 128, 256, 512) for y in (128, 256, 512)] +
           [(64, 128, 64), (64, 256, 256), (64, 512, 512), (256, 128, 128), (64, 64, 64),
            (18, 64, 64), (7, 32, 32)])
 
@@ -55,6 +55,34 @@ def test_transforms(dev, shape, prec):
             if flags & af.PRESERVE_INPUT:
                 assert rel_l2(sd.cpu().numpy(), s) < 1e-6
         p.destroy()
+
+
+@pytest.mark.parametrize("prec", ["f64", "f32"])
+@pytest.mark.parametrize("shape", SHAPES + [(32, 256, 512)])
+def test_c2c(dev, shape, prec):
+    """Both directions, two passes and one pass per axis, and a call whose
+    output is its input on the same plan."""
+    import torch
+    import accfft_amd as af
+    fp, rdt, cdt, tol = _t(prec)
+    x = rng(shape[1]).standard_normal(shape) + 1j * rng(9).standard_normal(shape)
+    xd = torch.tensor(x, dtype=cdt, device=dev)
+    out = torch.empty_like(xd)
+    p = af.Plan("c2c", shape, xd, out, fp, af.ACCFFT_ESTIMATE)
+    ref, inv = np.fft.fftn(x), np.fft.ifftn(x)
+    for choice in (-1, -2):
+        p.set_tuning(0, choice)
+        p.execute_c2c(af.ACCFFT_FORWARD, xd, out)
+        torch.cuda.synchronize()
+        assert rel_l2(out.cpu().numpy(), ref) < tol
+        p.execute_c2c(af.ACCFFT_BACKWARD, xd.clone(), out)
+        torch.cuda.synchronize()
+        assert rel_l2(out.cpu().numpy() / np.prod(shape), inv) < tol
+        same = xd.clone()
+        p.execute_c2c(af.ACCFFT_FORWARD, same, same)
+        torch.cuda.synchronize()
+        assert rel_l2(same.cpu().numpy(), ref) < tol
+    p.destroy()
 
 
 @pytest.mark.parametrize("prec", ["f64", "f32"])
