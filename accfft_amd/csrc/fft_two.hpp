@@ -207,12 +207,15 @@ struct TwoSym {
 
 // In place or out of place over [N0][N1][Nh]: a.Sin / a.Sout the x strides,
 // a.Din / a.Dout the n2 strides (R Nh), a.nlines = R Nh columns, a.tw the
-// full table of N0.  M_C2C: transforms of sign SIGN.  M_MULT: forward, the
+// full table of N0.  M_C2C: transforms of sign SIGN; FP64 has the forward
+// kernel alone, whose inverse is conj(F(conj x)) by flip as in mix_s_kernel
+// (its own inverse spilled 12 registers: 547 against 512 us at 512^3).
+// M_MULT: forward, the
 // symbol a.sym (a.Ch = Nh, a.C = R), inverse, the inverse running the
 // forward stages backwards.
 template <typename T, int N0, int M, int MODE, int SIGN>
 __global__ void __launch_bounds__((XYCfg<T, N0, M, MODE>::TPB), (MODE == M_MULT ? XYCfg<T, N0, M, MODE>::MULT_WAVES : 4))
-    two_xy_kernel(FftArgs<T> a) {
+    two_xy_kernel(FftArgs<T> a, unsigned flip) {
   using K = XYTile<T, N0, M, MODE>;
   constexpr int W = K::W, TPB = K::TPB, R0 = K::R0, R1 = K::R1, R2 = K::R2, L = K::L;
   static_assert(MODE == M_C2C || SIGN < 0, "M_MULT starts forward");
@@ -237,6 +240,13 @@ __global__ void __launch_bounds__((XYCfg<T, N0, M, MODE>::TPB), (MODE == M_MULT 
         v[i][r] = ld_global(at_off<const cpx<T>>(src + r * (N0 / R0) * a.Sin + i * a.Din, off));
   }
   K::stage_tw(tw, a.tw, t);
+  constexpr bool FLIP = MODE == M_C2C && sizeof(T) == 8;
+  if constexpr (FLIP) {
+#pragma unroll
+    for (int i = 0; i < M; ++i)
+#pragma unroll
+      for (int r = 0; r < R0; ++r) v[i][r] = conj_if(v[i][r], flip);
+  }
   auto w0 = [&](int i, int r) { return K::w0(t, i, r); };
   auto r1 = [&](int i, int r) { return K::r1(t, i, r); };
   auto w1 = [&](int i, int r) { return K::w1(t, i, r); };
@@ -258,7 +268,8 @@ __global__ void __launch_bounds__((XYCfg<T, N0, M, MODE>::TPB), (MODE == M_MULT 
       for (int i = 0; i < PER; ++i)
 #pragma unroll
         for (int r = 0; r < R; ++r)
-          *at_off<cpx<T>>(dst + (i * (TPB / L) + r * (N0 / R)) * a.Sout, off) = o[i][r];
+          *at_off<cpx<T>>(dst + (i * (TPB / L) + r * (N0 / R)) * a.Sout, off) =
+              FLIP ? conj_if(o[i][r], flip) : o[i][r];
     };
     if constexpr (R2 > 1) {
       typename K::V2 o;
