@@ -492,10 +492,11 @@ struct LayZ {
   __device__ __forceinline__ void map(int b, int nb, float rnb, int& line, int& j) const {
     line = fdivmod(b, nb, rnb, j);
   }
-  // (butterfly u, output q) of a prime stage: threads walk q fastest, so a
-  // wavefront reads the same inputs and writes neighbouring outputs
-  __device__ __forceinline__ void map_q(int b, int Q, float rq, int& u, int& q) const {
-    u = fdivmod(b, Q, rq, q);
+  // (butterfly u < per, output q < Q) of a prime stage: threads walk q
+  // fastest, so a wavefront reads the same inputs and writes neighbouring
+  // outputs
+  __device__ __forceinline__ void map_q(int b, int Q, int per, int& u, int& q) const {
+    u = fdivmod(b, Q, 1.0f / (float)Q, q);
   }
 };
 struct LayS {
@@ -505,11 +506,9 @@ struct LayS {
     j = b >> (__ffs(w) - 1);  // w is a power of two
     line = b & (w - 1);
   }
-  // columns fastest, then q
-  __device__ __forceinline__ void map_q(int b, int Q, float rq, int& u, int& q) const {
-    const int sh = __ffs(w) - 1;
-    const int j = fdivmod(b >> sh, Q, rq, q);
-    u = (j << sh) | (b & (w - 1));
+  // butterflies (columns) fastest, then q
+  __device__ __forceinline__ void map_q(int b, int Q, int per, int& u, int& q) const {
+    q = fdivmod(b, per, 1.0f / (float)per, u);
   }
 };
 
@@ -539,6 +538,72 @@ __device__ __forceinline__ void dstage(const cpx<T>* src, cpx<T>* dst, int N, in
     const int base = (j - k) * R + k;
 #pragma unroll
     for (int r = 0; r < R; ++r) dst[lay.addr(line, base + r * NS)] = v[r];
+  }
+}
+
+// Second sweep of dstage_prime: the output pairs q, R-q for q = q1, q1 + Q of
+// LB butterflies of one thread (root(m) = exp(-2 pi i m / R) serves all of
+// them; the inputs' and roots' positions move by additions).
+template <typename T, int SIGN, int LB, class Lay, typename ROOT>
+__device__ __forceinline__ void prime_outputs(const cpx<T>* src, cpx<T>* dst, int N, int R, int NS,
+                                              int nj, int Q, const Lay& lay, const ROOT& root) {
+  const int NB = N / R, H = (R - 1) / 2;
+  const float rnb = 1.0f / (float)NB, rns = 1.0f / (float)NS;
+  const int per = (nj + LB - 1) / LB, total = per * Q;
+  const int step = lay.addr(0, NB), ostep = lay.addr(0, NS);
+  for (int b = threadIdx.x; b < total; b += blockDim.x) {
+    int q1, u0;
+    lay.map_q(b, Q, per, u0, q1);
+    const int q2 = q1 + Q <= H ? q1 + Q : 0;
+    int px[LB], py[LB], po[LB];
+    cpx<T> c1[LB], c2[LB], s1[LB], s2[LB];
+#pragma unroll
+    for (int l = 0; l < LB; ++l) {
+      int u = u0 + l * per, line, j, k;
+      if (u >= nj) u = nj - 1;  // (computed twice, stored once)
+      lay.map(u, NB, rnb, line, j);
+      (void)fdivmod(j, NS, rns, k);
+      px[l] = lay.addr(line, j);
+      py[l] = px[l] + R * step;
+      po[l] = lay.addr(line, (j - k) * R + k);
+      c1[l] = c2[l] = src[px[l]];
+      s1[l] = s2[l] = cpx<T>{(T)0, (T)0};
+    }
+    int m1 = 0, m2 = 0;
+#pragma unroll 4
+    for (int r = 1; r <= H; ++r) {
+      m1 += q1;
+      m1 = m1 >= R ? m1 - R : m1;
+      m2 += q2;
+      m2 = m2 >= R ? m2 - R : m2;
+      const cpx<T> w1 = root(m1), w2 = root(m2);
+#pragma unroll
+      for (int l = 0; l < LB; ++l) {
+        px[l] += step;
+        py[l] -= step;
+        const cpx<T> x = src[px[l]], y = src[py[l]];
+        c1[l].x += x.x * w1.x;
+        c1[l].y += x.y * w1.x;
+        s1[l].x += y.x * w1.y;  // -sin
+        s1[l].y += y.y * w1.y;
+        c2[l].x += x.x * w2.x;
+        c2[l].y += x.y * w2.x;
+        s2[l].x += y.x * w2.y;
+        s2[l].y += y.y * w2.y;
+      }
+    }
+#pragma unroll
+    for (int l = 0; l < LB; ++l) {
+      if (u0 + l * per >= nj) continue;
+      // w.y = -sin, so the SIGN * i sin term is mul_si<-SIGN>
+      const cpx<T> t1 = mul_si<-SIGN>(s1[l]), t2 = mul_si<-SIGN>(s2[l]);
+      dst[po[l] + q1 * ostep] = cadd(c1[l], t1);
+      if (q1 > 0) dst[po[l] + (R - q1) * ostep] = csub(c1[l], t1);
+      if (q2 > 0) {
+        dst[po[l] + q2 * ostep] = cadd(c2[l], t2);
+        dst[po[l] + (R - q2) * ostep] = csub(c2[l], t2);
+      }
+    }
   }
 }
 
@@ -582,44 +647,16 @@ __device__ void dstage_prime(cpx<T>* src, cpx<T>* dst, int N, int R, int NS, int
     }
   }
   __syncthreads();
-  const int Q = (H + 2) / 2;  // values of q: u and u + Q
-  const int nj = nlines * NB, total = nj * Q;
-  const float rq = 1.0f / (float)Q;
-  for (int b = threadIdx.x; b < total; b += blockDim.x) {
-    int q1, u, line, j, k;
-    lay.map_q(b, Q, rq, u, q1);
-    lay.map(u, NB, rnb, line, j);
-    (void)fdivmod(j, NS, rns, k);
-    const int q2 = q1 + Q <= H ? q1 + Q : 0;
-    const cpx<T> v0 = src[lay.addr(line, j)];
-    cpx<T> c1 = v0, c2 = v0, s1 = {(T)0, (T)0}, s2 = {(T)0, (T)0};
-    int m1 = 0, m2 = 0;
-    for (int r = 1; r <= H; ++r) {
-      const cpx<T> x = src[lay.addr(line, j + r * NB)], y = src[lay.addr(line, j + (R - r) * NB)];
-      m1 += q1;
-      m1 = m1 >= R ? m1 - R : m1;
-      m2 += q2;
-      m2 = m2 >= R ? m2 - R : m2;
-      const cpx<T> w1 = roots != nullptr ? roots[m1] : twg[m1 * NB];
-      const cpx<T> w2 = roots != nullptr ? roots[m2] : twg[m2 * NB];
-      c1.x += x.x * w1.x;
-      c1.y += x.y * w1.x;
-      s1.x += y.x * w1.y;  // -sin
-      s1.y += y.y * w1.y;
-      c2.x += x.x * w2.x;
-      c2.y += x.y * w2.x;
-      s2.x += y.x * w2.y;
-      s2.y += y.y * w2.y;
-    }
-    const int base = (j - k) * R + k;
-    // w.y = -sin, so the SIGN * i sin term is mul_si<-SIGN>
-    const cpx<T> t1 = mul_si<-SIGN>(s1), t2 = mul_si<-SIGN>(s2);
-    dst[lay.addr(line, base + q1 * NS)] = cadd(c1, t1);
-    if (q1 > 0) dst[lay.addr(line, base + (R - q1) * NS)] = csub(c1, t1);
-    if (q2 > 0) {
-      dst[lay.addr(line, base + q2 * NS)] = cadd(c2, t2);
-      dst[lay.addr(line, base + (R - q2) * NS)] = csub(c2, t2);
-    }
+  // two butterflies a thread where that leaves every thread a task
+  const int nj = nlines * NB, Q = (H + 2) / 2;  // values of q: q1 and q1 + Q
+  const bool pair = (nj + 1) / 2 * Q >= (int)blockDim.x;
+  if (roots != nullptr) {
+    auto root = [roots](int m) { return roots[m]; };
+    if (pair) prime_outputs<T, SIGN, 2>(src, dst, N, R, NS, nj, Q, lay, root);
+    else prime_outputs<T, SIGN, 1>(src, dst, N, R, NS, nj, Q, lay, root);
+  } else {
+    auto root = [twg, NB](int m) { return twg[m * NB]; };
+    prime_outputs<T, SIGN, 1>(src, dst, N, R, NS, nj, Q, lay, root);
   }
 }
 
