@@ -19,15 +19,21 @@ hipError_t launch_n(bool strided, int mode, unsigned flip, FftArgs<T>& a, int64_
       default: return hipErrorNotSupported;
     }
   } else {
-    using CF = MixZ<T, N>;
-    const dim3 g((unsigned)((units + CF::L - 1) / CF::L)), b(CF::TPB);
+#define AFFT_MIXZ(MODE)                                                                        \
+  case MODE: {                                                                                 \
+    using CF = MixZ<T, N, MODE>;                                                               \
+    const dim3 g((unsigned)((units + CF::L - 1) / CF::L)), b(CF::TPB);                         \
+    hipLaunchKernelGGL((mix_z_kernel<T, N, MODE>), g, b, 0, st, a, flip);                      \
+    break;                                                                                     \
+  }
     switch (mode) {
-      case M_C2C: hipLaunchKernelGGL((mix_z_kernel<T, N, M_C2C>), g, b, 0, st, a, flip); break;
-      case M_R2C: hipLaunchKernelGGL((mix_z_kernel<T, N, M_R2C>), g, b, 0, st, a, flip); break;
-      case M_C2R: hipLaunchKernelGGL((mix_z_kernel<T, N, M_C2R>), g, b, 0, st, a, flip); break;
-      case M_DERIV: hipLaunchKernelGGL((mix_z_kernel<T, N, M_DERIV>), g, b, 0, st, a, flip); break;
+      AFFT_MIXZ(M_C2C)
+      AFFT_MIXZ(M_R2C)
+      AFFT_MIXZ(M_C2R)
+      AFFT_MIXZ(M_DERIV)
       default: return hipErrorNotSupported;
     }
+#undef AFFT_MIXZ
   }
   return hipGetLastError();
 }

@@ -129,22 +129,38 @@ constexpr int mix_twoff(const MixSched& m, int s) {  // twiddle table offset of 
 }
 constexpr int mix_twn(const MixSched& m) { return mix_twoff(m, m.s); }
 
-// Threads per block for L lines: a multiple of the wavefront up to 512 that holds at most `most` elements a thread and leaves the fewest
-// threads without a butterfly, summed over the stages by their work.
+// Work of a block of t threads and L lines, threads without a butterfly
+// included, summed over the stages.
+constexpr long mix_cost(const MixSched& m, int n, int l, int t) {
+  long c = 0;
+  for (int s = 0; s < m.s; ++s) {
+    const int b = n / m.r[s] * l;
+    c += (long)((b + t - 1) / t) * t * m.r[s];
+  }
+  return c;
+}
+// Threads per block for L lines: the multiple of the wavefront up to 512 that
+// holds at most `most` elements a thread and wastes least.
 constexpr int mix_tpb(const MixSched& m, int n, int l, int most) {
   int best = 0;
   long cost = 0;
   for (int t = 64; t <= 512; t += 64) {
     if (t < 512 && (long)n * l > (long)most * t) continue;
-    long c = 0;
-    for (int s = 0; s < m.s; ++s) {
-      const int b = n / m.r[s] * l;
-      c += (long)((b + t - 1) / t) * t * m.r[s];
-    }
+    const long c = mix_cost(m, n, l, t);
     if (!best || c * 100 < cost * 97) {
       best = t;
       cost = c;
     }
+  }
+  return best;
+}
+// Lines of a contiguous tile: of l / 2 ... 4 l / 3, those that waste least.
+constexpr int mix_lines(const MixSched& m, int n, int l, int most) {
+  int best = l;
+  for (int k = l / 2 > 2 ? l / 2 : 2; k <= l + l / 3 && k <= 32; ++k) {
+    const long c = mix_cost(m, n, k, mix_tpb(m, n, k, most)) * best;
+    const long b = mix_cost(m, n, best, mix_tpb(m, n, best, most)) * k;
+    if (c * 100 < b * 97) best = k;
   }
   return best;
 }
@@ -176,12 +192,17 @@ struct MixS {
 // 1694 us with two, 1949 with four lines a block, FP32 384^3 93 us with
 // three, 103 with six), 2304 elements up to 256 (200^3 FP64 27 us with
 // eleven lines, 31 with five).
-template <typename T, int N>
+// Derivative passes from 192 points, which spend their time in butterflies,
+// take the line count that leaves the fewest threads idle (256 points: eight
+// lines fill 128 threads, nine leave a quarter idle; FP32 32.6 -> 29.5 us,
+// 240 points 31.0 -> 26.2 us); the other passes and shorter lines are up to
+// 10 % faster with the idle threads, which share the loads and stores.
+template <typename T, int N, int MODE>
 struct MixZ {
   static constexpr int most = N > 256 ? 1152 : 2304;
-  static constexpr int L0 = most / N > 2 ? most / N : 2;
-  static constexpr int L = L0 > 32 ? 32 : L0;
+  static constexpr int L0 = most / N > 2 ? (most / N > 32 ? 32 : most / N) : 2;
   static constexpr int R0 = mix_sched<T>(N).r[0], E = sizeof(T) == 4 ? 12 : 8;
+  static constexpr int L = MODE == M_DERIV && N >= 192 ? mix_lines(mix_sched<T>(N), N, L0, R0 > E ? R0 : E) : L0;
   static constexpr int TPB = mix_tpb(mix_sched<T>(N), N, L, R0 > E ? R0 : E);
 };
 
@@ -584,9 +605,9 @@ __global__ void __launch_bounds__((MixS<T, N>::TPB))
 // M_C2C, M_R2C, M_C2R, M_DERIV of the z pass; a line of the real modes is a
 // pair of real lines.
 template <typename T, int N, int MODE>
-__global__ void __launch_bounds__((MixZ<T, N>::TPB))
+__global__ void __launch_bounds__((MixZ<T, N, MODE>::TPB))
     mix_z_kernel(FftArgs<T> a, unsigned flip) {
-  using CF = MixZ<T, N>;
+  using CF = MixZ<T, N, MODE>;
   using E = Mix<T, N, CF::L, CF::TPB, false>;
   using S0 = typename E::template St<0>;
   using SL = typename E::Last;
