@@ -114,6 +114,37 @@ __device__ __forceinline__ void dft8(cpx<T>* v) {
   v[7] = csub(e[3], o3);
 }
 
+// 16 = 2 x 8 (decimation in time)
+template <typename T, int SIGN>
+__device__ __forceinline__ void dft16(cpx<T>* v) {
+  const T c1 = (T)0.92387953251128675613;  // cos(pi/8)
+  const T s1 = (T)0.38268343236508977173;  // sin(pi/8)
+  const T c2 = (T)0.70710678118654752440;
+  cpx<T> e[8], o[8];
+#pragma unroll
+  for (int r = 0; r < 8; ++r) {
+    e[r] = v[2 * r];
+    o[r] = v[2 * r + 1];
+  }
+  dft8<T, SIGN>(e);
+  dft8<T, SIGN>(o);
+  // W16^k = cos(pi k/8) + SIGN*i*sin(pi k/8)
+  const T cw[8] = {(T)1, c1, c2, s1, (T)0, -s1, -c2, -c1};
+  const T sw[8] = {(T)0, s1, c2, c1, (T)1, c1, c2, s1};
+#pragma unroll
+  for (int k = 0; k < 8; ++k) {
+    cpx<T> t;
+    if (k == 0) t = o[0];
+    else if (k == 4) t = mul_si<SIGN>(o[4]);
+    else {
+      const T wr = cw[k], wi = SIGN * sw[k];
+      t = {o[k].x * wr - o[k].y * wi, o[k].x * wi + o[k].y * wr};
+    }
+    v[k] = cadd(e[k], t);
+    v[k + 8] = csub(e[k], t);
+  }
+}
+
 // v exp(SIGN 2 pi i m / 32), m a constant after unrolling: quarter turns cost
 // no arithmetic, odd eighths two products of a sum.
 template <int SIGN, typename T>
@@ -134,8 +165,10 @@ __device__ __forceinline__ cpx<T> rot32(cpx<T> v, int m) {
 }
 
 // 16 = 4 x 4 and 32 = 8 x 4 (n = B n1 + n2, k = k1 + 4 k2, n1, k1 < 4): one
-// level of rotations between the two (16 as 2 x 8, which has two, is less
-// accurate and takes more products).
+// level of rotations between the two; 16 as 2 x 8 above has two, is less
+// accurate and takes more products.  For the kernels of fft_mix.hpp and
+// fft_two.hpp; the tiles of fft_kernels.hpp, whose persistent forms sit at
+// their register limit, lose 1.4 % with it (2048-point slab share).
 template <typename T, int B, int SIGN>
 __device__ __forceinline__ void dft4xB(cpx<T>* v) {
   cpx<T> y[4][B];
@@ -155,7 +188,7 @@ __device__ __forceinline__ void dft4xB(cpx<T>* v) {
   }
 }
 template <typename T, int SIGN>
-__device__ __forceinline__ void dft16(cpx<T>* v) { dft4xB<T, 4, SIGN>(v); }
+__device__ __forceinline__ void dft16q(cpx<T>* v) { dft4xB<T, 4, SIGN>(v); }
 template <typename T, int SIGN>
 __device__ __forceinline__ void dft32(cpx<T>* v) { dft4xB<T, 8, SIGN>(v); }
 

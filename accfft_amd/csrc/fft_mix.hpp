@@ -65,6 +65,7 @@ __device__ __forceinline__ void mdft(cpx<T>* v) {
   else if constexpr (R == 12) dft_pfa<T, 4, 3, SIGN>(v);
   else if constexpr (R == 14) dft_pfa<T, 2, 7, SIGN>(v);
   else if constexpr (R == 15) dft_pfa<T, 3, 5, SIGN>(v);
+  else if constexpr (R == 16) dft16q<T, SIGN>(v);
   else dft<T, R, SIGN>(v);
 }
 

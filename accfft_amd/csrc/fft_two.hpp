@@ -30,6 +30,7 @@ __device__ __forceinline__ gptr<V> at_off(B* base, uint32_t off) {
 template <typename T, int R, int SIGN>
 __device__ __forceinline__ void pdft(cpx<T>* v) {
   if constexpr (R == 1) return;
+  else if constexpr (R == 16) dft16q<T, SIGN>(v);
   else if constexpr (R == 32) dft32<T, SIGN>(v);
   else dft<T, R, SIGN>(v);
 }
