@@ -74,7 +74,9 @@ inline bool pair_mode(int mode) { return mode == M_R2C || mode == M_C2R || mode 
 // Tiles of the dynamic engine.  A launch of few blocks is bound by the
 // latency of one block's stages, so tiles are halved while the launch has
 // fewer than dyn_blocks blocks (one for each CU) and a tile keeps whole
-// 64-byte row segments (strided) or one line (z).
+// 64-byte row segments (strided) or one line (z).  Small mixed-radix grids
+// (40 us round trips) gained 1.2-1.57x; two blocks for each CU slowed a
+// 120 x 200 x 75 FP32 pair from 97 to 100 us.
 constexpr int64_t dyn_blocks = 256;
 inline int dyn_lines(int n, int64_t units) {
   int l = 2048 / n;
@@ -208,8 +210,9 @@ inline bool wide_tiles(int n) {
 }
 
 // Two-level strided C2C tiles (sfft4_kernel): on by default where they were
-// measured faster on MI355X (FP32 512, 1024, 2048; FP64 512 is faster with
-// the one-level tiles).  For measurement, ACCFFT_AMD_S4 (bit log2(n): use
+// measured faster on MI355X than the one-level ones (FP32 512, 1024, 2048;
+// FP64 512 is faster with the one-level tiles); plain 512-point C2C rows take
+// the mixed-radix kernels first (mix_pow2).  For measurement, ACCFFT_AMD_S4 (bit log2(n): use
 // them) overrides that choice and ACCFFT_AMD_S4V ("n:v,n:v", e.g.
 // "2048:2,1024:3") picks the configuration variant of a length.
 inline unsigned env_mask(const char* name, unsigned dflt) {

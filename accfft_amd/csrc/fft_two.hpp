@@ -8,11 +8,19 @@
 //   pass 2 (two_xy)  for each column (k1, kz): the M-point DFT over n2
 //                    (rows k1 + R n2 -> k1 + R k2, in place) and the x
 //                    transform.
-// Each pass transforms about sqrt(N0 N1 N2 / 2) points of every column at
-// once, 64 to 256 KiB a workgroup, held in registers (a CU has 512 KiB of
-// them); the LDS only exchanges real, then imaginary parts between stages.
-// Against one pass per axis this reads and writes the spectrum once less in
-// each direction: R + 3 C bytes instead of R + 5 C.
+// A workgroup transforms 16 to 256 KiB of a pass at once, held in registers
+// (a CU has 512 KiB of them); the LDS only exchanges real, then imaginary
+// parts between stages.  Against one pass per axis this reads and writes the
+// spectrum once less in each direction: R + 3 C bytes instead of R + 5 C.
+//
+// What bounds them (512^3 FP32, a large copy runs at 5.1 TB/s): pass 1 runs
+// at 5.1 TB/s (209 / 212 us r2c / c2r, two workgroups of 512 threads per CU);
+// pass 2 at 3.85-4.2 TB/s (279 / 259 us): one 256 KiB tile fills a CU, so
+// its 10 us of vector and 3 us of LDS time a tile are not hidden, and a copy
+// with its access pattern (64-byte segments of 4096 rows) reaches 4.5 TB/s.
+// One pass per axis takes 181 + 169 + 203 us forward.  Staggered starts of
+// the workgroups and 32-byte segments with two workgroups per CU measured no
+// faster.
 #pragma once
 #include "fft_mix.hpp"
 
@@ -213,7 +221,8 @@ struct TwoSym {
 // (its own inverse spilled 12 registers: 547 against 512 us at 512^3).
 // M_MULT: forward, the
 // symbol a.sym (a.Ch = Nh, a.C = R), inverse, the inverse running the
-// forward stages backwards.
+// forward stages backwards (512^3 FP32 425 us, against 171 + 232 + 181 us as
+// y, fused x and y passes; 256^3 42 against 25 + 30 + 24 us).
 template <typename T, int N0, int M, int MODE, int SIGN>
 __global__ void __launch_bounds__((XYCfg<T, N0, M, MODE>::TPB), (MODE == M_MULT ? XYCfg<T, N0, M, MODE>::MULT_WAVES : 4))
     two_xy_kernel(FftArgs<T> a, unsigned flip) {

@@ -444,9 +444,10 @@ def run_ops(steps):
     solve) and the differentiable loss 1/2 |div(grad(invlap u)) - g|^2 at
     256^3 FP32 with its adjoint backward.  Bytes are this library's passes
     (each operand read and written once per pass): grad 3 x 2R (one fused
-    per-axis derivative pass per component), the spectral operators 2R + 8C
-    (z r2c, y, x forward + symbol + inverse in one pass, y, z c2r),
-    divergence 8R (2R + two accumulating passes of 3R)."""
+    per-axis derivative pass per component), the spectral operators 2R + 4C
+    (z and most of y, the rest of y with x and the symbol forward and back,
+    and the first pass inverted), the Poisson solve 2R + 8C (one pass per
+    axis), divergence 8R (2R + two accumulating passes of 3R)."""
     import torch
     import accfft_amd as af
     from accfft_amd import autograd as ag
@@ -464,9 +465,9 @@ def run_ops(steps):
     out = {}
     ops = [
         ("grad_3_components", lambda: plan.grad(u, o[0], o[1], o[2]), 6 * R),
-        ("laplace", lambda: plan.laplace(u, o[0]), 2 * R + 8 * C),
-        ("inv_laplace", lambda: plan.inv_laplace(u, o[0]), 2 * R + 8 * C),
-        ("biharmonic", lambda: plan.biharmonic(u, o[0]), 2 * R + 8 * C),
+        ("laplace", lambda: plan.laplace(u, o[0]), 2 * R + 4 * C),
+        ("inv_laplace", lambda: plan.inv_laplace(u, o[0]), 2 * R + 4 * C),
+        ("biharmonic", lambda: plan.biharmonic(u, o[0]), 2 * R + 4 * C),
         ("poisson_solve", lambda: plan.poisson_solve(u, o[0], 1), 2 * R + 8 * C),
     ]
     div = torch.empty_like(u)

@@ -191,7 +191,11 @@ int accfft_amd_plan_info(const accfft_amd_plan* plan, int n[3], int isize[3],
  * transform (N1 = 8 M, M = 16 ... 256, N2 = 256 ... 2048, not split),
  * get reports -3 on the y axis when that fusion is off; set(1, -3) turns
  * it off (separate z and N1-point y passes, tuned as above) and
- * set(1, -1) restores it. */
+ * set(1, -1) restores it.
+ * Out-of-place r2c and c2c plans on power-of-two grids up to 512 points a
+ * side run their full transforms in two passes over memory, which have one
+ * configuration; a choice other than -1 on the x or y axis (or -3) takes
+ * the plan back to one pass per axis. */
 int accfft_amd_plan_get_tuning(const accfft_amd_plan* plan, int choice[3]);
 int accfft_amd_plan_set_tuning(accfft_amd_plan* plan, int axis, int choice);
 /* Default data pointers recorded at plan time (src/accfft_gpu.cpp:447-450). */
