@@ -212,9 +212,10 @@ inline bool wide_tiles(int n) {
 // Two-level strided C2C tiles (sfft4_kernel): on by default where they were
 // measured faster on MI355X than the one-level ones (FP32 512, 1024, 2048;
 // FP64 512 is faster with the one-level tiles); plain 512-point C2C rows take
-// the mixed-radix kernels first (mix_pow2).  For measurement, ACCFFT_AMD_S4 (bit log2(n): use
-// them) overrides that choice and ACCFFT_AMD_S4V ("n:v,n:v", e.g.
-// "2048:2,1024:3") picks the configuration variant of a length.
+// the mixed-radix kernels first (mix_pow2).  For measurement, ACCFFT_AMD_S4
+// (bit log2(n): use them) overrides that choice and ACCFFT_AMD_S4V
+// ("n:v,n:v", e.g. "2048:2,1024:3") picks the configuration variant of a
+// length.
 inline unsigned env_mask(const char* name, unsigned dflt) {
   const char* e = sweep_env(name);
   return e ? (unsigned)strtoul(e, nullptr, 0) : dflt;

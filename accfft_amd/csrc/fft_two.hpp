@@ -28,8 +28,9 @@ namespace afft {
 
 // Element at 32-bit byte offset `off` of a uniform base: the base stays in
 // scalar registers (scalar arithmetic for the row steps) and a thread keeps
-// one offset register for all of its loads.  The grids of this file are at
-// most 512^3 FP64 spectra, 2.2 GB.
+// one offset register for all of its loads.  Pass 1 has a 64-bit base for
+// each plane (at most 4 MB of offsets); pass 2 spans the grid, at most a
+// 512^3 FP64 spectrum, 2.2 GB.
 template <typename V, typename B>
 __device__ __forceinline__ gptr<V> at_off(B* base, uint32_t off) {
   return (gptr<V>)((gptr<typename std::conditional<std::is_const<B>::value, const char, char>::type>)base + off);
@@ -582,8 +583,9 @@ __device__ __forceinline__ void split_factors(cpx<T>* te, cpx<T>* to, const cpx<
 //   E_q[k] = (U_q[k] + conj U_-q[-k]) / 2, O_q[k] = -i (U_q[k] - conj U_-q[-k]) / 2
 // are the transforms of the even and odd rows, and the last radix-2 level
 //   X_q = E_q + w_R^q O_q, X_{q+P} = E_q - w_R^q O_q
-// rides on the split, with the twiddles of the M-point level in its factors.  a.idist / a.odist: row pitches, a.Din / a.Dout plane
-// strides, a.C = M, a.tw / twy the full tables of NZ and N1.
+// rides on the split, with the twiddles of the M-point level in its factors.
+// a.idist / a.odist: row pitches, a.Din / a.Dout plane strides, a.C = M,
+// a.tw / twy the full tables of NZ and N1.
 template <typename T, int NZ, int R>
 __global__ void __launch_bounds__((ZYCfg<T, R / 2, NZ>::TPB))
     two_zy_r2c_kernel(FftArgs<T> a, const cpx<T>* __restrict__ twy) {
