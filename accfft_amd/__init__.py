@@ -149,6 +149,16 @@ def _check(status: int, what: str) -> None:
 _raw_stream = None
 
 
+def _forget_stream():
+    """A forked child may not use its parent's device: its next call goes
+    through torch.cuda.current_stream() again, which raises there."""
+    global _raw_stream
+    _raw_stream = None
+
+
+os.register_at_fork(after_in_child=_forget_stream)
+
+
 def _stream():
     """torch's current stream on the current device, as an address.  Read
     through torch's raw accessors: the Stream object that
