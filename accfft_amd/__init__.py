@@ -368,7 +368,14 @@ class Plan:
     def execute_r2c(self, data=None, data_out=None, timer=None, xyz: int = 7):
         arr, tp = self._timer(timer)
         out_b = self._out_bytes if xyz & 4 else 0
-        _check(lib().accfft_amd_execute_r2c(self._bind(), self._a(data, self._in_bytes, "r2c input"),
+        # without the z transform the y and x transforms run in place on the
+        # input (the plan's own for None), as rows of n[2]//2+1 complex
+        in_b = self._in_bytes
+        if not xyz & 4 and xyz & 3:
+            in_b = max(in_b, self._out_bytes)
+            if data is None:
+                data = self._keep[0]
+        _check(lib().accfft_amd_execute_r2c(self._bind(), self._a(data, in_b, "r2c input"),
                                             self._a(data_out, out_b, "r2c output"), tp, xyz),
                "execute_r2c")
         self._untimer(timer, arr)
