@@ -433,9 +433,11 @@ int accfft_amd_plan_set_tuning(accfft_amd_plan* p, int axis, int choice) {
   }
   if (p->fp == ACCFFT_AMD_F32) {
     p->tf[axis].s4v = choice;
+    p->tf[axis].forced = choice != -1;
     p->tf[axis].xg = -1;
   } else {
     p->td[axis].s4v = choice;
+    p->td[axis].forced = choice != -1;
     p->td[axis].xg = -1;
   }
   return ACCFFT_AMD_OK;

@@ -39,6 +39,8 @@ struct AxisTab {
   // strided C2C configuration picked by the plan's MEASURE tuning: -1 the
   // built-in rule, -2 one-level tiles, v >= 0 two-level variant S4Cfg<T, n, v>
   int s4v = -1;
+  // s4v was set by hand (accfft_amd_plan_set_tuning), not by timing
+  bool forced = false;
   // tiles per XCD chunk picked by the tuning (xcd_tile's g); -1 the rule
   int xg = -1;
   // the plan's tile queue of the persistent strided tiles (QUEUE_WORDS
@@ -438,11 +440,20 @@ hipError_t launch_mix(bool strided, int mode, int sign, FftArgs<T> a, const Axis
 // 240-250 us).  z up to 128 points (64^3 FP64 8.5 -> 6.6 us) and the FP32
 // derivative at 256 and 512 (37 -> 32, 276 -> 217 us); the other z passes are
 // faster as they are (256^3 FP64 r2c 60 against 69 us, 512^3 369 against 410
-// us).  A plan's tuned choice (s4v) comes first.
+// us).
 template <typename T>
 inline bool mix_pow2(int n, bool strided, int mode) {
   if (strided) return n <= 256 || (n == 512 && (sizeof(T) == 8 || mode == M_C2C));
   return n <= 128 || (sizeof(T) == 4 && mode == M_DERIV && n <= 512);
+}
+// Whether a pass of a power-of-two axis goes to them.  A choice made by hand
+// (s4v) comes first in every mode; one that MEASURE made timed the C2C tiles
+// and speaks for those alone (512-point FP64 multiply 423 us here, 569 us on
+// the tile a C2C timing may prefer).
+template <typename T>
+inline bool mix_first(const AxisTab<T>& tab, bool strided, int mode) {
+  if (!tab.tw_mix || !tab.is_static || !mix_pow2<T>(tab.n, strided, mode)) return false;
+  return tab.s4v == -1 || (!tab.forced && (mode == M_MULT || mode == M_DERIV));
 }
 
 // Launch one axis pass.  strided = false: contiguous lines (z layout).
@@ -456,7 +467,7 @@ hipError_t launch_fft(bool strided, int mode, int sign, FftArgs<T> a, const Axis
   const int64_t units = pair_mode(mode) ? (a.nlines + 1) / 2 : a.nlines;
   if (units <= 0) return hipSuccess;
   const size_t csz = sizeof(cpx<T>);
-  if (tab.tw_mix && tab.is_static && tab.s4v == -1 && mix_pow2<T>(n, strided, mode)) {
+  if (mix_first(tab, strided, mode)) {
     const hipError_t e = launch_mix<T>(strided, mode, sign, a, tab, st);
     if (e != hipErrorNotSupported) return e;
   }
