@@ -421,11 +421,13 @@ struct Ops {
   }
 
   // ---------------------------------------------------------- two passes
-  // 1 x 1 r2c and c2c plans on power-of-two grids (fft_two.hpp).  A tuning choice on
-  // the x or y axis, or the separate z and y passes (choice -3), takes the
-  // plan back to one pass per axis.
+  // 1 x 1 r2c and c2c plans on power-of-two grids (fft_two.hpp).  A tuning
+  // choice on the y axis, on the x axis where pass 2 is not the plain x pass
+  // (M > 1), or the separate z and y passes (choice -3) take the plan back to
+  // one pass per axis.
   static bool two(const accfft_amd_plan* p) {
-    return p->two && tab(p, 0).s4v == -1 && tab(p, 1).s4v == -1 && (ysub(p).n == 0 || p->yfuse);
+    return p->two && tab(p, 1).s4v == -1 && (p->n[1] == p->two || tab(p, 0).s4v == -1) &&
+           (ysub(p).n == 0 || p->yfuse);
   }
   // pass 1, real <-> half spectrum rows k1 + R n2; adjw as in the z passes
   static int two_zy(accfft_amd_plan* p, int sign, const void* in, void* out, int adjw = 0) {
@@ -1236,19 +1238,27 @@ struct Ops {
   // rule stays.  As with FFTW's MEASURE, the choice can change results in
   // the last bits.  Split-precision plans time their own (matrix-core)
   // tiles the same way.
-  static int tune(accfft_amd_plan* p) {
+  struct TunePass {
+    int ax, order;
+    FftArgs<T> a;
+    int64_t in_elems, out_elems;
+  };
+  // The passes that are timed: those of the full transforms.  The two-pass
+  // kernels have one configuration; with M = 1 pass 2 is the plain x pass.
+  // Calls on such plans that run one pass per axis (masks, Poisson solves,
+  // inverse biharmonic, a c2c whose output is its input) keep the built-in
+  // rule on the 512-point axes of a plan with M > 1: timing them took 58 to
+  // 300 ms at plan creation (512^3) and gained nothing (rule / what MEASURE
+  // picks: c2c in place FP32 1193 / 1187 us, FP64 2459 / 2467 us, x and y alone
+  // 862 / 855 and 1754 / 1762 us; for r2c it picks the rule).
+  static std::vector<TunePass> tune_passes(accfft_amd_plan* p) {
     const int64_t N0 = p->n[0], N1 = p->n[1], N2 = p->n[2], Nh = N2 / 2 + 1;
-    struct Pass {
-      int ax, order;
-      FftArgs<T> a;
-      int64_t in_elems, out_elems;
-    };
-    std::vector<Pass> passes;
-    if (two(p)) return ACCFFT_AMD_OK;  // its passes have one configuration
+    std::vector<TunePass> passes;
     if (p->kind == 1 || p->kind == 2) {
       const int64_t L = p->kind == 1 ? Nh : N2, e = N0 * N1 * L;
-      if (!yfused(p)) passes.push_back({1, 1, y_args(p, nullptr, nullptr, L), e, 0});
-      passes.push_back({0, 2, x_args(p, nullptr, nullptr, L), e, 0});
+      const bool tp = two(p);
+      if (!tp && !yfused(p)) passes.push_back({1, 1, y_args(p, nullptr, nullptr, L), e, 0});
+      if (!tp || N1 == p->two) passes.push_back({0, 2, x_args(p, nullptr, nullptr, L), e, 0});
     } else if (p->kind == 3) {
       const int P = p->nprocs;
       const int64_t n0 = N0 / P, n1 = N1 / P, Np = ws_pitch(Nh);
@@ -1258,9 +1268,13 @@ struct Ops {
       passes.push_back({0, 2, sargs(nullptr, nullptr, n1 * Nh, n1 * Nh, 0, 0, n1 * Nh, n1 * Nh),
                         N0 * n1 * Nh, 0});
     }
+    return passes;
+  }
+  static int tune(accfft_amd_plan* p) {
+    const std::vector<TunePass> passes = tune_passes(p);
     int64_t elems = 0;
     bool any = false;
-    for (const Pass& q : passes) {
+    for (const TunePass& q : passes) {
       const AxisTab<T>& t = tab(p, q.ax);
       if (!t.is_static || !t.tw_sub || (t.n != 512 && t.n != 1024 && t.n != 2048)) continue;
       any = true;
@@ -1277,7 +1291,7 @@ struct Ops {
     if (hipMemsetAsync(buf, 0, (size_t)elems * sizeof(C), p->stream) != hipSuccess ||
         hipEventCreate(&e0) != hipSuccess || hipEventCreate(&e1) != hipSuccess)
       st = ACCFFT_AMD_ERR_HIP;
-    for (const Pass& q : passes) {
+    for (const TunePass& q : passes) {
       if (st) break;
       AxisTab<T>& t = const_cast<AxisTab<T>&>(tab(p, q.ax));
       if (!t.is_static || !t.tw_sub || (t.n != 512 && t.n != 1024 && t.n != 2048)) continue;

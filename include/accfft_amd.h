@@ -192,10 +192,17 @@ int accfft_amd_plan_info(const accfft_amd_plan* plan, int n[3], int isize[3],
  * get reports -3 on the y axis when that fusion is off; set(1, -3) turns
  * it off (separate z and N1-point y passes, tuned as above) and
  * set(1, -1) restores it.
- * Out-of-place r2c and c2c plans on power-of-two grids up to 512 points a
- * side run their full transforms in two passes over memory, which have one
- * configuration; a choice other than -1 on the x or y axis (or -3) takes
- * the plan back to one pass per axis. */
+ * Out-of-place 1 x 1 r2c and c2c plans run their full transforms in two
+ * passes over memory when N1 and N2 are powers of two from 32 to 512 and N0
+ * is one too or N1 <= 64 (c2c tiles of at most 256 KiB and grids with enough
+ * blocks: two_rows and two_rows_c2c in csrc/fft_two_launch.hpp).  Pass 1 and,
+ * for N1 > 64, pass 2 have one configuration: MEASURE times only an x pass
+ * that is pass 2 as it stands (N1 = 32 or 64; FP64 c2c with N2 = 512: 32),
+ * and calls of the other plans
+ * that run one pass per axis (masks, Poisson solves, inverse biharmonic, c2c
+ * with in == out) keep the built-in rule.  A choice other than -1 on the y
+ * axis, on the x axis where N1 > 64, or -3, takes the plan back to one pass
+ * per axis. */
 int accfft_amd_plan_get_tuning(const accfft_amd_plan* plan, int choice[3]);
 int accfft_amd_plan_set_tuning(accfft_amd_plan* plan, int axis, int choice);
 /* Default data pointers recorded at plan time (src/accfft_gpu.cpp:447-450). */

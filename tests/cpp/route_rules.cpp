@@ -40,10 +40,45 @@ void choices(const char* prec) {
                (int)mix_first(axis<T>(512, s4v, forced), true, modes[m]));
 }
 
+// an out-of-place 1 x 1 plan (kind 1 r2c, 2 c2c)
+template <typename T>
+accfft_amd_plan plan(int kind, int n0, int n1, int n2) {
+  accfft_amd_plan p;
+  p.kind = kind;
+  p.n[0] = n0;
+  p.n[1] = n1;
+  p.n[2] = n2;
+  p.fp = sizeof(T) == 4 ? ACCFFT_AMD_F32 : ACCFFT_AMD_F64;
+  for (int ax = 0; ax < 3; ++ax) const_cast<AxisTab<T>&>(Ops<T>::tab(&p, ax)) = axis<T>(p.n[ax]);
+  p.two = kind == 1 ? two_rows(p.n) : two_rows_c2c<T>(p.n);
+  return p;
+}
+// two-pass form with no choice, with one on x, with one on y; timed axes
+template <typename T>
+void tuning(const char* prec, int kind, int n0, int n1, int n2) {
+  accfft_amd_plan p = plan<T>(kind, n0, n1, n2);
+  printf("tune_%s_%d_%dx%dx%d two %d", prec, kind, n0, n1, n2, (int)Ops<T>::two(&p));
+  for (int ax = 0; ax < 2; ++ax) {
+    auto& t = const_cast<AxisTab<T>&>(Ops<T>::tab(&p, ax));
+    t.s4v = -2;
+    printf(" %d", (int)Ops<T>::two(&p));
+    t.s4v = -1;
+  }
+  printf(" axes");
+  for (const auto& q : Ops<T>::tune_passes(&p)) printf(" %d", q.ax);
+  printf("\n");
+}
+
 }  // namespace
 
 int main() {
   choices<float>("f32");
   choices<double>("f64");
+  tuning<float>("f32", 1, 2048, 64, 512);
+  tuning<double>("f64", 1, 512, 32, 256);
+  tuning<float>("f32", 2, 1024, 64, 64);
+  tuning<double>("f64", 2, 512, 64, 512);
+  tuning<float>("f32", 1, 512, 512, 512);
+  tuning<double>("f64", 1, 512, 512, 500);
   return 0;
 }
