@@ -50,7 +50,7 @@ accfft_amd_plan plan(int kind, int n0, int n1, int n2) {
   p.n[2] = n2;
   p.fp = sizeof(T) == 4 ? ACCFFT_AMD_F32 : ACCFFT_AMD_F64;
   for (int ax = 0; ax < 3; ++ax) const_cast<AxisTab<T>&>(Ops<T>::tab(&p, ax)) = axis<T>(p.n[ax]);
-  p.two = kind == 1 ? two_rows(p.n) : two_rows_c2c<T>(p.n);
+  p.two = kind == 1 ? two_rows<T>(p.n) : two_rows_c2c<T>(p.n);
   return p;
 }
 // two-pass form with no choice, with one on x, with one on y; timed axes
@@ -69,9 +69,22 @@ void tuning(const char* prec, int kind, int n0, int n1, int n2) {
   printf("\n");
 }
 
+// rows of pass 1, r2c and c2c
+template <typename T>
+void rows(const char* prec, int n0, int n1, int n2) {
+  const int n[3] = {n0, n1, n2};
+  printf("rows_%s_%dx%dx%d %d %d\n", prec, n0, n1, n2, two_rows<T>(n), two_rows_c2c<T>(n));
+}
+
 }  // namespace
 
 int main() {
+  for (int n0 : {1, 15, 16, 31, 32, 63, 64, 512})
+    for (int n1 : {32, 64, 128})
+      for (int n2 : {32, 128, 256, 512}) {
+        rows<float>("f32", n0, n1, n2);
+        rows<double>("f64", n0, n1, n2);
+      }
   choices<float>("f32");
   choices<double>("f64");
   tuning<float>("f32", 1, 2048, 64, 512);

@@ -48,3 +48,25 @@ def test_measure_times_the_passes_of_the_transform(rules):
     for key in ("f64_2_512x64x512", "f32_1_512x512x512"):
         assert rules["tune_" + key] == "two 1 0 0 axes", key
     assert rules["tune_f64_1_512x512x500"] == "two 0 0 0 axes 1 0"
+
+
+def test_large_pass_1_tiles_need_blocks(rules):
+    """Tiles of 128 KiB and more, and of 512-point lines, run in two passes
+    from as many x planes as the tile has complex rows."""
+    def rows(prec, n0, n1, n2):
+        return tuple(int(v) for v in rules[f"rows_{prec}_{n0}x{n1}x{n2}"].split())
+    for prec in ("f32", "f64"):
+        for n0 in (1, 15, 31, 32, 512):  # small tiles: any number of planes
+            assert rows(prec, n0, 64, 32) == (64, 64)
+        # real rows of 512 points: 16 (32 rows) and 32 (64 rows) blocks
+        assert rows(prec, 15, 32, 512)[0] == 0 and rows(prec, 16, 32, 512)[0] == 32
+        assert rows(prec, 31, 64, 512)[0] == 0 and rows(prec, 32, 64, 512)[0] == 64
+        assert rows(prec, 31, 32, 512)[1] == 0 and rows(prec, 32, 32, 512)[1] == 32
+        assert rows(prec, 512, 128, 512)[0] == 64
+    # 256 points: FP32 r2c tiles of 64 rows are 64 KiB, FP64 ones 128 KiB
+    assert rows("f32", 1, 64, 256) == (64, 0)
+    assert rows("f64", 31, 64, 256) == (0, 0) and rows("f64", 32, 64, 256) == (64, 0)
+    assert rows("f32", 63, 64, 256) == (64, 0) and rows("f32", 64, 64, 256) == (64, 64)
+    assert rows("f64", 1, 64, 128) == (64, 0) and rows("f64", 64, 64, 128) == (64, 64)
+    # FP64 complex rows of 512 points: 32 at a time, two blocks a plane
+    assert rows("f64", 32, 64, 512)[1] == 32
