@@ -440,19 +440,44 @@ hipError_t launch_mix(bool strided, int mode, int sign, FftArgs<T> a, const Axis
 // 240-250 us).  z up to 128 points (64^3 FP64 8.5 -> 6.6 us) and the FP32
 // derivative at 256 and 512 (37 -> 32, 276 -> 217 us); the other z passes are
 // faster as they are (256^3 FP64 r2c 60 against 69 us, 512^3 369 against 410
-// us).
+// us).  This is the largest set; C2C passes up to 256 points and z passes up
+// to 128 follow mix_pow2 below.
 template <typename T>
-inline bool mix_pow2(int n, bool strided, int mode) {
+constexpr bool mix_pow2_built(int n, bool strided, int mode) {
   if (strided) return n <= 256 || (n == 512 && (sizeof(T) == 8 || mode == M_C2C));
   return n <= 128 || (sizeof(T) == 4 && mode == M_DERIV && n <= 512);
+}
+// Lines this short cost these kernels partial cache lines: a z block loads
+// N / R0 adjacent points at a time (and each c2r element twice), a strided
+// one 128-byte segments, which rows that are not multiples of 128 bytes split
+// over two lines.  The memory-side cache (256 MB) hides it until the pass is
+// large, the later the longer the line; from there on the tiles of
+// fft_kernels.hpp, which move whole lines and wider segments, are faster (us,
+// here / there: z c2r FP32 2048 x 2048 x 16 210 / 124, 1024 x 1024 x 64 183 /
+// 104, FP64 2048 x 1024 x 32 307 / 193, 512 x 512 x 64 52 / 44; z derivatives
+// FP32 2048 x 1024 x 32 175 / 98; y C2C FP64 1024 x 32 x 513 94-100 / 82, FP32
+// 512 x 64 x 513 52-55 / 49, x C2C FP64 128 x 256 x 1024 242 / 210).  Below the
+// line: FP32 z c2r 256 x 256 x 64 8.0 / 9.6, y C2C 512 x 64 x 129 12 / 14, FP64
+// 256 x 64 x 129 11-12 / 15.  Fused strided passes are faster at every size
+// measured (to 2^26 points).
+template <typename T>
+inline bool mix_pow2(const FftArgs<T>& a, int n, bool strided, int mode) {
+  if (!mix_pow2_built<T>(n, strided, mode)) return false;
+  if (strided ? mode != M_C2C || n > 256 : n > 128) return true;
+  const bool real = !strided && mode != M_C2C;
+  const int64_t es = real ? sizeof(T) : sizeof(cpx<T>);
+  const bool whole = !real && (!strided || (a.Sin | a.Sout) * es % 128 == 0);
+  const int64_t line = (int64_t)n * n * (whole ? 128 : 32) << 10;
+  const int64_t cap = real ? (int64_t)256 << 20 : n < 256 ? es << 25 : (int64_t)1 << 30;
+  return 2 * a.nlines * n * es <= (line < cap ? line : cap);
 }
 // Whether a pass of a power-of-two axis goes to them.  A choice made by hand
 // (s4v) comes first in every mode; one that MEASURE made timed the C2C tiles
 // and speaks for those alone (512-point FP64 multiply 423 us here, 569 us on
 // the tile a C2C timing may prefer).
 template <typename T>
-inline bool mix_first(const AxisTab<T>& tab, bool strided, int mode) {
-  if (!tab.tw_mix || !tab.is_static || !mix_pow2<T>(tab.n, strided, mode)) return false;
+inline bool mix_first(const FftArgs<T>& a, const AxisTab<T>& tab, bool strided, int mode) {
+  if (!tab.tw_mix || !tab.is_static || !mix_pow2(a, tab.n, strided, mode)) return false;
   return tab.s4v == -1 || (!tab.forced && (mode == M_MULT || mode == M_DERIV));
 }
 
@@ -467,7 +492,7 @@ hipError_t launch_fft(bool strided, int mode, int sign, FftArgs<T> a, const Axis
   const int64_t units = pair_mode(mode) ? (a.nlines + 1) / 2 : a.nlines;
   if (units <= 0) return hipSuccess;
   const size_t csz = sizeof(cpx<T>);
-  if (mix_first(tab, strided, mode)) {
+  if (mix_first(a, tab, strided, mode)) {
     const hipError_t e = launch_mix<T>(strided, mode, sign, a, tab, st);
     if (e != hipErrorNotSupported) return e;
   }

@@ -28,6 +28,29 @@ AxisTab<T> axis(int n, int s4v = -1, bool forced = false) {
   return t;
 }
 
+// nlines lines; strided: rows of `row` elements
+template <typename T>
+FftArgs<T> pass(int n, int64_t nlines, int64_t row = 512) {
+  FftArgs<T> a{};
+  a.nlines = nlines;
+  a.C = a.Sin = a.Sout = row;
+  a.Din = a.Dout = n * row;
+  return a;
+}
+// log2 of the most points (2^15 ... 2^27) of a pass over lines of n points
+// that goes to the mixed-radix kernels, 0 for none; rows of a multiple of 128
+// bytes, and of one element more
+template <typename T>
+void most(const char* prec, int n) {
+  for (int strided = 0; strided < 2; ++strided)
+    for (int mode : {M_C2C, M_R2C, M_C2R, M_DERIV, M_MULT})
+      for (int odd = 0; odd < 2; ++odd) {
+        int lg = 27;
+        while (lg >= 15 && !mix_first(pass<T>(n, ((int64_t)1 << lg) / n, 512 + odd), axis<T>(n), strided, mode)) --lg;
+        printf("most_%s_%d_%c%d_%d %d\n", prec, n, strided ? 's' : 'z', mode, odd, lg < 15 ? 0 : lg);
+      }
+}
+
 // a 512-point strided axis on the mixed-radix kernels
 template <typename T>
 void choices(const char* prec) {
@@ -37,7 +60,7 @@ void choices(const char* prec) {
     for (int forced = 0; forced < 2; ++forced)
       for (int m = 0; m < 3; ++m)
         printf("mix512_%s_%s_%d_%d %d\n", prec, names[m], s4v, forced,
-               (int)mix_first(axis<T>(512, s4v, forced), true, modes[m]));
+               (int)mix_first(pass<T>(512, 512 * 512), axis<T>(512, s4v, forced), true, modes[m]));
 }
 
 // an out-of-place 1 x 1 plan (kind 1 r2c, 2 c2c)
@@ -79,6 +102,11 @@ void rows(const char* prec, int n0, int n1, int n2) {
 }  // namespace
 
 int main() {
+  printf("modes %d %d %d %d %d\n", M_C2C, M_R2C, M_C2R, M_DERIV, M_MULT);
+  for (int n : {16, 32, 64, 128, 256, 512, 1024}) {
+    most<float>("f32", n);
+    most<double>("f64", n);
+  }
   for (int n0 : {1, 15, 16, 31, 32, 63, 64, 512})
     for (int n1 : {32, 64, 128})
       for (int n2 : {32, 128, 256, 512}) {

@@ -70,3 +70,29 @@ def test_large_pass_1_tiles_need_blocks(rules):
     assert rows("f64", 1, 64, 128) == (64, 0) and rows("f64", 64, 64, 128) == (64, 64)
     # FP64 complex rows of 512 points: 32 at a time, two blocks a plane
     assert rows("f64", 32, 64, 512)[1] == 32
+
+
+def test_large_passes_of_short_power_of_two_lines(rules):
+    """The mixed-radix kernels take power-of-two z and C2C passes up to the
+    bytes from which the wider tiles are faster, and fused strided passes of
+    any size.  Entries: log2 of the most points (27: any), 0 never."""
+    c2c, r2c, c2r, deriv, mult = rules["modes"].split()
+    n = (16, 32, 64, 128, 256, 512, 1024)
+
+    def row(prec, kind, mode, odd=0):
+        return tuple(int(rules[f"most_{prec}_{v}_{kind}{mode}_{odd}"]) for v in n)
+    for odd in (0, 1):
+        for mode in (r2c, c2r):
+            assert row("f32", "z", mode, odd) == (20, 22, 24, 25, 0, 0, 0)
+            assert row("f64", "z", mode, odd) == (19, 21, 23, 24, 0, 0, 0)
+        assert row("f32", "z", deriv, odd) == (20, 22, 24, 25, 27, 27, 0)
+        assert row("f64", "z", deriv, odd) == (19, 21, 23, 24, 0, 0, 0)
+        assert row("f32", "z", c2c, odd) == (21, 23, 24, 24, 0, 0, 0)
+        assert row("f64", "z", c2c, odd) == (20, 22, 24, 24, 0, 0, 0)
+        assert row("f32", "s", deriv, odd) == (27, 27, 27, 27, 27, 0, 0)
+        for mode in (mult, deriv):
+            assert row("f64", "s", mode, odd) == (27, 27, 27, 27, 27, 27, 0)
+    assert row("f32", "s", c2c, 0) == (21, 23, 24, 24, 26, 27, 0)
+    assert row("f32", "s", c2c, 1) == (19, 21, 23, 24, 26, 27, 0)
+    assert row("f64", "s", c2c, 0) == (20, 22, 24, 24, 25, 27, 0)
+    assert row("f64", "s", c2c, 1) == (18, 20, 22, 24, 25, 27, 0)
