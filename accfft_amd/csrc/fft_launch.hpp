@@ -430,23 +430,6 @@ hipError_t launch_mix(bool strided, int mode, int sign, FftArgs<T> a, const Axis
   }
 }
 
-// Powers of two on the mixed-radix kernels.  Strided up to 256 points: one
-// or two LDS round trips instead of three or four (64^3 FP64 passes 9.0-10
-// -> 6.5-7.2 us, 256^3 FP32 x pass 29 -> 26 us, multiply 47 -> 30 us,
-// derivatives 38 -> 28 us, FP64 51 -> 47, 81 -> 54, 65-69 -> 52-56 us); 512
-// points FP64 (multiply 569 -> 423 us, derivatives 751 / 512 -> 570 / 407
-// us, C2C 401-418 -> 388-394 us) and FP32 C2C (204 / 197 -> 197 / 184 us; the
-// fused FP32 passes stay with the two-level tiles, derivatives 219 against
-// 240-250 us).  z up to 128 points (64^3 FP64 8.5 -> 6.6 us) and the FP32
-// derivative at 256 and 512 (37 -> 32, 276 -> 217 us); the other z passes are
-// faster as they are (256^3 FP64 r2c 60 against 69 us, 512^3 369 against 410
-// us).  This is the largest set; C2C passes up to 256 points and z passes up
-// to 128 follow mix_pow2 below.
-template <typename T>
-constexpr bool mix_pow2_built(int n, bool strided, int mode) {
-  if (strided) return n <= 256 || (n == 512 && (sizeof(T) == 8 || mode == M_C2C));
-  return n <= 128 || (sizeof(T) == 4 && mode == M_DERIV && n <= 512);
-}
 // Lines this short cost these kernels partial cache lines: a z block loads
 // N / R0 adjacent points at a time (and each c2r element twice), a strided
 // one 128-byte segments, which rows that are not multiples of 128 bytes split

@@ -6,36 +6,44 @@
 namespace afft {
 namespace {
 
+// the powers of two have the passes that launch_fft sends here
+template <typename T, int N>
+constexpr bool built(bool strided, int mode) {
+  return (N & (N - 1)) != 0 || mix_pow2_built<T>(N, strided, mode);
+}
+
 template <typename T, int N>
 hipError_t launch_n(bool strided, int mode, unsigned flip, FftArgs<T>& a, int64_t units,
                     hipStream_t st) {
   if (strided) {
-    using CF = MixS<T, N>;
-    const dim3 g((unsigned)((units + CF::L - 1) / CF::L)), b(CF::TPB);
-    switch (mode) {
-      case M_C2C: hipLaunchKernelGGL((mix_s_kernel<T, N, M_C2C>), g, b, 0, st, a, flip); break;
-      case M_MULT: hipLaunchKernelGGL((mix_s_kernel<T, N, M_MULT>), g, b, 0, st, a, flip); break;
-      case M_DERIV: hipLaunchKernelGGL((mix_s_kernel<T, N, M_DERIV>), g, b, 0, st, a, flip); break;
-      default: return hipErrorNotSupported;
+#define AFFT_MIXS(MODE)                                                                         \
+  if constexpr (built<T, N>(true, MODE))                                                        \
+    if (mode == MODE) {                                                                         \
+      using CF = MixS<T, N>;                                                                    \
+      const dim3 g((unsigned)((units + CF::L - 1) / CF::L)), b(CF::TPB);                        \
+      hipLaunchKernelGGL((mix_s_kernel<T, N, MODE>), g, b, 0, st, a, flip);                     \
+      return hipGetLastError();                                                                 \
     }
+    AFFT_MIXS(M_C2C)
+    AFFT_MIXS(M_MULT)
+    AFFT_MIXS(M_DERIV)
+#undef AFFT_MIXS
   } else {
-#define AFFT_MIXZ(MODE)                                                                        \
-  case MODE: {                                                                                 \
-    using CF = MixZ<T, N, MODE>;                                                               \
-    const dim3 g((unsigned)((units + CF::L - 1) / CF::L)), b(CF::TPB);                         \
-    hipLaunchKernelGGL((mix_z_kernel<T, N, MODE>), g, b, 0, st, a, flip);                      \
-    break;                                                                                     \
-  }
-    switch (mode) {
-      AFFT_MIXZ(M_C2C)
-      AFFT_MIXZ(M_R2C)
-      AFFT_MIXZ(M_C2R)
-      AFFT_MIXZ(M_DERIV)
-      default: return hipErrorNotSupported;
+#define AFFT_MIXZ(MODE)                                                                         \
+  if constexpr (built<T, N>(false, MODE))                                                       \
+    if (mode == MODE) {                                                                         \
+      using CF = MixZ<T, N, MODE>;                                                              \
+      const dim3 g((unsigned)((units + CF::L - 1) / CF::L)), b(CF::TPB);                        \
+      hipLaunchKernelGGL((mix_z_kernel<T, N, MODE>), g, b, 0, st, a, flip);                     \
+      return hipGetLastError();                                                                 \
     }
+    AFFT_MIXZ(M_C2C)
+    AFFT_MIXZ(M_R2C)
+    AFFT_MIXZ(M_C2R)
+    AFFT_MIXZ(M_DERIV)
 #undef AFFT_MIXZ
   }
-  return hipGetLastError();
+  return hipErrorNotSupported;
 }
 
 }  // namespace

@@ -2,6 +2,7 @@
 fft_two_launch.hpp and exec.hpp, evaluated on the CPU by
 tests/cpp/route_rules.cpp."""
 import os
+import re
 import shutil
 import subprocess
 
@@ -96,3 +97,26 @@ def test_large_passes_of_short_power_of_two_lines(rules):
     assert row("f32", "s", c2c, 1) == (19, 21, 23, 24, 26, 27, 0)
     assert row("f64", "s", c2c, 0) == (20, 22, 24, 24, 25, 27, 0)
     assert row("f64", "s", c2c, 1) == (18, 20, 22, 24, 25, 27, 0)
+
+
+def test_every_mixed_radix_kernel_is_reached(rules):
+    """The library holds the kernels of the list's lengths that a pass can
+    be sent to, and no others."""
+    import accfft_amd as af
+    nm = shutil.which("nm")
+    if nm is None or not os.path.exists(af.LIB_PATH):
+        pytest.skip("needs nm and the built library")
+    syms = subprocess.run([nm, "-C", af.LIB_PATH], check=True, capture_output=True, text=True).stdout
+    have = {(k, t, int(n), m) for k, t, n, m in re.findall(
+        r" afft::mix_([sz])_kernel<(float|double), (\d+), (\d)>", syms)}
+    lists = open(os.path.join(HERE, "..", "accfft_amd", "csrc", "fft_mix_list.hpp")).read()
+    lengths = [int(v) for v in re.findall(r"X\((\d+)\)", lists.split("#define AFFT_MIX_EACH")[0])]
+    c2c, r2c, c2r, deriv, mult = rules["modes"].split()
+    want = set()
+    for t, prec in (("float", "f32"), ("double", "f64")):
+        for n in lengths:
+            for kind, modes in (("s", (c2c, mult, deriv)), ("z", (c2c, r2c, c2r, deriv))):
+                for m in modes:
+                    if n & (n - 1) or int(rules[f"most_{prec}_{n}_{kind}{m}_0"]):
+                        want.add((kind, t, n, m))
+    assert have == want
