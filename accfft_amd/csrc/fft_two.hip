@@ -63,7 +63,9 @@ hipError_t launch_two_xy<AFFT_T>(int mode, int sign, int n0, int m, const FftArg
   if (n0 == NN && m == MM) {                                                                      \
     using CF = XYCfg<AFFT_T, NN, MM, M_C2C>;                                                      \
     using CM = XYCfg<AFFT_T, NN, MM, M_MULT>;                                                     \
-    const dim3 g((unsigned)((a.nlines + CF::W - 1) / CF::W)), b(mode == M_C2C ? CF::TPB : CM::TPB); \
+    static_assert(CF::W == CM::W, "one tile width");                                              \
+    if (a.nlines % CF::W) return hipErrorNotSupported;                                            \
+    const dim3 g((unsigned)(a.nlines / CF::W)), b(mode == M_C2C ? CF::TPB : CM::TPB);             \
     constexpr int INV = sizeof(AFFT_T) == 4 ? +1 : -1;  /* FP64: the forward kernel, conjugated */  \
     const unsigned flip = sign > 0 ? 0x80000000u : 0u;                                            \
     if (mode == M_C2C && sign < 0) hipLaunchKernelGGL((two_xy_kernel<AFFT_T, NN, MM, M_C2C, -1>), g, b, 0, st, a, flip); \

@@ -8,7 +8,7 @@
 //   pass 2 (two_xy)  for each column (k1, kz): the M-point DFT over n2
 //                    (rows k1 + R n2 -> k1 + R k2, in place) and the x
 //                    transform.
-// A workgroup transforms 16 to 256 KiB of a pass at once, held in registers
+// A workgroup transforms 4 to 256 KiB of a pass at once, held in registers
 // (a CU has 512 KiB of them); the LDS only exchanges real, then imaginary
 // parts between stages.  Against one pass per axis this reads and writes the
 // spectrum once less in each direction: R + 3 C bytes instead of R + 5 C.
@@ -29,8 +29,9 @@ namespace afft {
 // Element at 32-bit byte offset `off` of a uniform base: the base stays in
 // scalar registers (scalar arithmetic for the row steps) and a thread keeps
 // one offset register for all of its loads.  Pass 1 has a 64-bit base for
-// each plane (at most 4 MB of offsets); pass 2 spans the grid, at most a
-// 512^3 FP64 spectrum, 2.2 GB.
+// each plane (at most 4 MB of offsets); in pass 2 the offsets span the grid,
+// at most 1.08 GB (the 512^3 half spectrum in FP64; c2c 1.07 GB, 512^3 in
+// FP32 and 512 x 256 x 512 in FP64).
 template <typename V, typename B>
 __device__ __forceinline__ gptr<V> at_off(B* base, uint32_t off) {
   return (gptr<V>)((gptr<typename std::conditional<std::is_const<B>::value, const char, char>::type>)base + off);
@@ -236,13 +237,11 @@ __global__ void __launch_bounds__((XYCfg<T, N0, M, MODE>::TPB), (MODE == M_MULT 
   int64_t tile = xcd_tile(blockIdx.x, gridDim.x, (unsigned)a.xgroup);
   if (a.reverse) tile = (int64_t)gridDim.x - 1 - tile;
   const int64_t col0 = tile * W;
-  const int cols = a.nlines - col0 < W ? (int)(a.nlines - col0) : W;  // of this tile
-  // first-stage registers: column t % W (clamped: a column past the last
-  // one repeats it and is not stored), x = t / W + r N0 / R0, all n2
+  // first-stage registers: column t % W, x = t / W + r N0 / R0, all n2 (every
+  // tile is whole: the launcher refuses R Nh columns that W does not divide)
   typename K::V0 v;
   {
-    const int c = t % W < cols ? t % W : cols - 1;
-    const uint32_t off = (uint32_t)((c + (t / W) * a.Sin) * sizeof(cpx<T>));
+    const uint32_t off = (uint32_t)((t % W + (t / W) * a.Sin) * sizeof(cpx<T>));
     const cpx<T>* src = reinterpret_cast<const cpx<T>*>(a.in) + col0;
 #pragma unroll
     for (int r = 0; r < R0; ++r)
@@ -272,7 +271,6 @@ __global__ void __launch_bounds__((XYCfg<T, N0, M, MODE>::TPB), (MODE == M_MULT 
   if constexpr (MODE == M_C2C) {
     auto store = [&](auto& o, auto per, auto rad) {
       constexpr int PER = decltype(per)::value, R = decltype(rad)::value;
-      if (line % W >= cols) return;
       cpx<T>* dst = reinterpret_cast<cpx<T>*>(a.out) + col0;
       const uint32_t off = (uint32_t)((line % W + (line / W) * a.Dout + (t / L) * a.Sout) * sizeof(cpx<T>));
 #pragma unroll
@@ -333,7 +331,6 @@ __global__ void __launch_bounds__((XYCfg<T, N0, M, MODE>::TPB), (MODE == M_MULT 
     K::template stage<K::P1, R1, K::NS1, +1, true>(x, tb, tw);
     K::exchange(x, v, buf, R2 > 1, br1, bw0);
     K::template first<+1>(v);
-    if (tb % W >= cols) return;
     cpx<T>* dst = reinterpret_cast<cpx<T>*>(a.out) + col0;
     const uint32_t off = (uint32_t)((tb % W + (tb / W) * a.Sout) * sizeof(cpx<T>));
 #pragma unroll

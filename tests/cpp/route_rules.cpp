@@ -5,6 +5,7 @@
 
 #include "../../accfft_amd/csrc/dispatch.hpp"
 #include "../../accfft_amd/csrc/exec.hpp"
+#include "../../accfft_amd/csrc/fft_two.hpp"
 
 using namespace afft;
 
@@ -99,9 +100,41 @@ void rows(const char* prec, int n0, int n1, int n2) {
   printf("rows_%s_%dx%dx%d %d %d\n", prec, n0, n1, n2, two_rows<T>(n), two_rows_c2c<T>(n));
 }
 
+// columns of pass 2 that its tiles would leave over, and bytes its offsets
+// span, over every plan of x length N0 that has one
+template <typename T, int N0, int M>
+void pass2(const char* prec) {
+  int64_t left = 0, bytes = 0;
+  int plans = 0;
+  for (int kind = 1; kind < 3; ++kind)
+    for (int n1 = 32; n1 <= 512; n1 *= 2)
+      for (int n2 = 32; n2 <= 512; n2 *= 2) {
+        const int n[3] = {N0, n1, n2};
+        const int r = kind == 1 ? two_rows<T>(n) : two_rows_c2c<T>(n);
+        if (!r || n1 / r != M) continue;
+        const int64_t nh = kind == 1 ? n2 / 2 + 1 : n2;
+        left += r * nh % XYCfg<T, N0, M, M_C2C>::W;
+        bytes = std::max(bytes, (int64_t)N0 * n1 * nh * (int64_t)sizeof(cpx<T>));
+        ++plans;
+      }
+  printf("pass2_%s_%d_%d %d %lld %lld\n", prec, N0, M, plans, (long long)left, (long long)bytes);
+}
+template <typename T>
+void pass2(const char* prec) {
+#define AFFT_N0(N) pass2<T, N, 2>(prec), pass2<T, N, 4>(prec), pass2<T, N, 8>(prec)
+  AFFT_N0(32);
+  AFFT_N0(64);
+  AFFT_N0(128);
+  AFFT_N0(256);
+  AFFT_N0(512);
+#undef AFFT_N0
+}
+
 }  // namespace
 
 int main() {
+  pass2<float>("f32");
+  pass2<double>("f64");
   printf("modes %d %d %d %d %d\n", M_C2C, M_R2C, M_C2R, M_DERIV, M_MULT);
   for (int n : {16, 32, 64, 128, 256, 512, 1024}) {
     most<float>("f32", n);

@@ -120,3 +120,17 @@ def test_every_mixed_radix_kernel_is_reached(rules):
                     if n & (n - 1) or int(rules[f"most_{prec}_{n}_{kind}{m}_0"]):
                         want.add((kind, t, n, m))
     assert have == want
+
+
+def test_pass_2_tiles_are_whole(rules):
+    """Every plan's pass 2 has a whole number of tiles (the kernel has no
+    guard, its launcher refuses others), and its 32-bit byte offsets reach
+    the whole grid."""
+    most = 0
+    for prec in ("f32", "f64"):
+        for n0 in (32, 64, 128, 256, 512):
+            for m in (2, 4, 8):
+                plans, left, span = map(int, rules[f"pass2_{prec}_{n0}_{m}"].split())
+                assert plans > 0 and left == 0 and span < 2 ** 32
+                most = max(most, span)
+    assert most == 512 * 512 * 257 * 16  # the 512^3 half spectrum in FP64
