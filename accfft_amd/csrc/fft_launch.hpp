@@ -439,9 +439,12 @@ hipError_t launch_mix(bool strided, int mode, int sign, FftArgs<T> a, const Axis
 // here / there: z c2r FP32 2048 x 2048 x 16 210 / 124, 1024 x 1024 x 64 183 /
 // 104, FP64 2048 x 1024 x 32 307 / 193, 512 x 512 x 64 52 / 44; z derivatives
 // FP32 2048 x 1024 x 32 175 / 98; y C2C FP64 1024 x 32 x 513 94-100 / 82, FP32
-// 512 x 64 x 513 52-55 / 49, x C2C FP64 128 x 256 x 1024 242 / 210).  Below the
+// 512 x 64 x 513 52-55 / 49, x C2C FP64 128 x 256 x 1024 242 / 210, FP32 pairs 64
+// x 256 x 1024 102 / 93).  Below the
 // line: FP32 z c2r 256 x 256 x 64 8.0 / 9.6, y C2C 512 x 64 x 129 12 / 14, FP64
-// 256 x 64 x 129 11-12 / 15.  Fused strided passes are faster at every size
+// 128 x 64 x 513 26 / 29.  The column blocks of a pencil share move it down for
+// the z passes (c2r FP32 512 x 512 x 64 46.8 / 34.3, 512 x 256 x 128 46.6 / 38.3,
+// 256 x 512 x 64 16.4 / 19.9).  Fused strided passes are faster at every size
 // measured (to 2^26 points).
 template <typename T>
 inline bool mix_pow2(const FftArgs<T>& a, int n, bool strided, int mode) {
@@ -449,9 +452,10 @@ inline bool mix_pow2(const FftArgs<T>& a, int n, bool strided, int mode) {
   if (strided ? mode != M_C2C || n > 256 : n > 128) return true;
   const bool real = !strided && mode != M_C2C;
   const int64_t es = real ? sizeof(T) : sizeof(cpx<T>);
-  const bool whole = !real && (!strided || (a.Sin | a.Sout) * es % 128 == 0);
-  const int64_t line = (int64_t)n * n * (whole ? 128 : 32) << 10;
-  const int64_t cap = real ? (int64_t)256 << 20 : n < 256 ? es << 25 : (int64_t)1 << 30;
+  const bool whole = (a.Sin | a.Sout) * es % 128 == 0;  // rows
+  const int64_t per = strided ? (whole ? es / 2 : 4) : mode == M_C2C ? 16 : mode == M_DERIV ? 8 : 4;
+  const int64_t line = n * n * es * per << 10;
+  const int64_t cap = real ? (int64_t)(a.zcol ? 64 : 256) << 20 : n < 256 ? es << 25 : (int64_t)1 << 30;
   return 2 * a.nlines * n * es <= (line < cap ? line : cap);
 }
 // Whether a pass of a power-of-two axis goes to them.  A choice made by hand

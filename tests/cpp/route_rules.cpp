@@ -31,8 +31,9 @@ AxisTab<T> axis(int n, int s4v = -1, bool forced = false) {
 
 // nlines lines; strided: rows of `row` elements
 template <typename T>
-FftArgs<T> pass(int n, int64_t nlines, int64_t row = 512) {
+FftArgs<T> pass(int n, int64_t nlines, int64_t row = 512, int64_t zcol = 0) {
   FftArgs<T> a{};
+  a.zcol = zcol;
   a.nlines = nlines;
   a.C = a.Sin = a.Sout = row;
   a.Din = a.Dout = n * row;
@@ -40,14 +41,14 @@ FftArgs<T> pass(int n, int64_t nlines, int64_t row = 512) {
 }
 // log2 of the most points (2^15 ... 2^27) of a pass over lines of n points
 // that goes to the mixed-radix kernels, 0 for none; rows of a multiple of 128
-// bytes, and of one element more
+// bytes, of one element more, and (z) half-spectrum columns in blocks
 template <typename T>
 void most(const char* prec, int n) {
   for (int strided = 0; strided < 2; ++strided)
     for (int mode : {M_C2C, M_R2C, M_C2R, M_DERIV, M_MULT})
-      for (int odd = 0; odd < 2; ++odd) {
+      for (int odd = 0; odd < 3; ++odd) {
         int lg = 27;
-        while (lg >= 15 && !mix_first(pass<T>(n, ((int64_t)1 << lg) / n, 512 + odd), axis<T>(n), strided, mode)) --lg;
+        while (lg >= 15 && !mix_first(pass<T>(n, ((int64_t)1 << lg) / n, 512 + odd % 2, odd / 2 * 9), axis<T>(n), strided, mode)) --lg;
         printf("most_%s_%d_%c%d_%d %d\n", prec, n, strided ? 's' : 'z', mode, odd, lg < 15 ? 0 : lg);
       }
 }
