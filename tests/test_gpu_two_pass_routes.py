@@ -124,3 +124,33 @@ def test_planes(dev, shape, r2c, c2c, prec):
     assert rel_l2(c.cpu().numpy() / np.prod(shape), a) < 2 * tol
     p.destroy()
     q.destroy()
+
+
+@pytest.mark.parametrize("prec", ["f64", "f32"])
+@pytest.mark.parametrize("shape", [(512, 64, 128), (1024, 32, 64), (2048, 64, 32)])
+def test_choices_of_the_x_pass(dev, shape, prec):
+    """Where pass 2 is the plain x pass, MEASURE and every choice on x keep
+    the two passes and their results."""
+    import torch
+    import accfft_amd as af
+    fp, rdt, cdt, tol = _t(prec)
+    a = rng(shape[0]).standard_normal(shape)
+    x = torch.tensor(a, dtype=rdt, device=dev)
+    h = torch.empty(shape[:2] + (shape[2] // 2 + 1,), dtype=cdt, device=dev)
+    back = torch.empty_like(x)
+    ref = np.fft.rfftn(a)
+    p = af.Plan("r2c", shape, x, h, fp, af.ACCFFT_MEASURE)
+    chosen = p.tuning()
+    assert chosen[0] in (-1, -2, 0, 1, 2, 3) and chosen[1:] == (-1, -1)
+    for choice in (chosen[0], -2, -1, 0, 1, 2, 3):
+        try:
+            p.set_tuning(0, choice)
+        except af.AccfftError:
+            continue  # no such variant of this length and precision
+        names = _kinds(p, lambda: p.execute_r2c(x, h))
+        assert len(names) == 2 and any("_zy" in k for k in names), names
+        assert rel_l2(h.cpu().numpy(), ref) < tol, choice
+        p.execute_c2r(h, back)
+        torch.cuda.synchronize()
+        assert rel_l2(back.cpu().numpy() / np.prod(shape), a) < 2 * tol, choice
+    p.destroy()
