@@ -14,11 +14,13 @@
 // ([n][L], lanes along the columns), contiguous ones whole lines
 // ([line][n], lanes along the line).
 //
-// The passes are bound by memory: 384^3 FP32 84 / 85 / 76 us (z, y, x; 5.4 to
-// 6.0 TB/s, a large copy reaches 5.1 and part of the reads come from the
-// memory-side cache) against 207 / 81-140 us in the run-time engine; 768^3
-// FP64 1.32 / 1.43 / 1.56 ms (4.7-5.5 TB/s).  Small grids are bound by the
-// latency of one block's stages and the launch (64^3 passes 6.4 us).
+// The passes are bound by memory: 384^3 FP32 z r2c 84, y 82-87, x 76 us (5.2
+// to 6.0 TB/s, a large copy reaches 5.1 and part of the reads come from the
+// memory-side cache) and z c2r 100 us (4.5 TB/s; it loads each element of the
+// half spectrum twice, for k and N - k) against 207 / 81-140 / 216 us in the
+// run-time engine; 768^3 FP64 z r2c 1.34, y and x 1.41-1.53 ms (4.8-5.4 TB/s).
+// Small grids are bound by the latency of one block's stages and the launch
+// (64^3 FP64 x passes 4.3 us).
 //
 // LDS layout: one pad row (element) after every R0 = first radix, when R0
 // is even.  The first stage writes with a stride of R0 rows, which padded is

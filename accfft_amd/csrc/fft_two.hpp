@@ -220,10 +220,11 @@ struct TwoSym {
 // a.Din / a.Dout the n2 strides (R Nh), a.nlines = R Nh columns, a.tw the
 // full table of N0.  M_C2C: transforms of sign SIGN; FP64 has the forward
 // kernel alone, whose inverse is conj(F(conj x)) by flip as in mix_s_kernel
-// (its own inverse spilled 12 registers: 547 against 512 us at 512^3).
+// (its own inverse spilled 12 registers: 547 against 512 us at 512^3; 465-487
+// us since the kernel has no guard for a partial tile).
 // M_MULT: forward, the
 // symbol a.sym (a.Ch = Nh, a.C = R), inverse, the inverse running the
-// forward stages backwards (512^3 FP32 425 us, against 171 + 232 + 181 us as
+// forward stages backwards (512^3 FP32 418 us, against 171 + 232 + 181 us as
 // y, fused x and y passes; 256^3 42 against 25 + 30 + 24 us).
 template <typename T, int N0, int M, int MODE, int SIGN>
 __global__ void __launch_bounds__((XYCfg<T, N0, M, MODE>::TPB), (MODE == M_MULT ? XYCfg<T, N0, M, MODE>::MULT_WAVES : 4))

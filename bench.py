@@ -647,6 +647,8 @@ def main():
             f"  x{cnt}")
 
     alg, comp = alg_bytes_roundtrip(n, 4)
+    # what this library's own passes read and write, each element once per pass
+    moved = sum(b * cnt for _, cnt, b in prof.values()) / args.steps
     # dominant kernel = largest total time in the profiled pass
     dom = max(prof.items(), key=lambda kv: kv[1][0])
     dname, (dtot, dcnt, dbytes) = dom
@@ -697,6 +699,8 @@ def main():
             "roundtrip_rel_l2": err,
             "pass_model_bytes": alg,
             "pass_model_frac_of_hbm_peak": round(alg / (ms * 1e-3) / 1e9 / HBM_PEAK_GBS, 4),
+            "moved_bytes": moved,
+            "moved_frac_of_hbm_peak": round(moved / (ms * 1e-3) / 1e9 / HBM_PEAK_GBS, 4),
             "compulsory_frac_of_hbm_peak": round(comp / (ms * 1e-3) / 1e9 / HBM_PEAK_GBS, 4),
             "device_copy_GBps": round(copy_gbps, 1),
             "tile_tuning_xyz": tuning,
